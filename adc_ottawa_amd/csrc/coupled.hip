@@ -321,7 +321,7 @@ void CoupledPrecon::form_schur(double s, Prec bp) {
     // pair tensors of P C^T e_j straight from the integral blocks, then the
     // down contractions: A0 e_j = H11 e_j - C P C^T e_j (P from orbital
     // energies; with ADC(2)-x the half sigma-vectors below use hii)
-    Hd.ensure_lowprec(bp);
+    Hd.ensure_pairs(bp);
     const size_t es = bp == Prec::F64 ? 8 : (bp == Prec::F32 ? 4 : 2);
     Hd.ZG.alloc((size_t)n1 * n1 * nc * es);
     const double* V = (const double*)Hd.is[0].V.get();

@@ -110,35 +110,114 @@ size_t Handle::integral_bytes(Prec p) const {
   return prec_size(p) * 2 * ((size_t)d.v * d.v + (size_t)d.o * d.o) * (size_t)d.n1;
 }
 
-// FP64 integral blocks of the INT form, assembled from the factors by GEMMs:
-// V[(a,c)][bl] = sum_P Bvv[P][a][c] Bov[P][bl], O[(k,m)][bl] = sum_P
-// Boo[P][k][m] Bov[P][bl]; Vt and Ot are the same numbers in the layouts the
-// up contractions read.
+// FP64 integral block assembled from the factors: V[(a,c)][bl] = sum_P
+// Bvv[P][a][c] Bov[P][bl] (virt) or O[(k,m)][bl] = sum_P Boo[P][k][m]
+// Bov[P][bl].
+void Handle::integral_block(bool virt, DevBuf<char>& out) {
+  const int64_t n1 = d.n1;
+  const int r = virt ? d.v : d.o;
+  out.alloc(sizeof(double) * r * r * n1);
+  GemmArgs g;
+  g.M = r * r; g.N = (int)n1; g.K = d.naux;
+  g.A = virt ? (const void*)Bvv.get() : (const void*)Boo.get();
+  g.sam = 1; g.sak = (int64_t)r * r;
+  g.B = Bov.get(); g.sbk = n1; g.sbn = 1;
+  g.map.C = out.get();
+  g.map.scm = n1; g.map.scn = 1;
+  gemm(g, Prec::F64, gws, st);
+}
+
+// Operands of the CSF form in precision p, each rounded once from the FP64
+// blocks (which are kept only when the pair-tensor form has built them).
+void Handle::build_csf(Prec p) {
+  CsfSet& c = cs[p == Prec::F64 ? 0 : 1];
+  if (c.ready) return;
+  DevBuf<char> tV, tO;
+  const char* V = is[0].V.get();
+  if (!is[0].ready) {
+    integral_block(true, tV);
+    V = tV.get();
+  }
+  if (!cs_O.get()) {
+    const char* O = is[0].O.get();
+    if (!is[0].ready) {
+      integral_block(false, tO);
+      O = tO.get();
+    }
+    cs_O.alloc(csf_o_elems(dk));
+    launch_csf_build_o((const double*)O, dk, cs_O.get(), st);
+    cs_zeros.alloc(csf_zeros(dk));
+    HIP_CHECK(hipMemsetAsync(cs_zeros.get(), 0, sizeof(double) * csf_zeros(dk), st));
+  }
+  if (p == Prec::F64) {
+    c.V.alloc(sizeof(double) * csf_v_elems<double>(dk));
+    launch_csf_build_v<double>((const double*)V, dk, (double*)c.V.get(), st);
+  } else {
+    c.V.alloc(sizeof(float) * csf_v_elems<float>(dk));
+    launch_csf_build_v<float>((const double*)V, dk, (float*)c.V.get(), st);
+  }
+  HIP_CHECK(hipStreamSynchronize(st));
+  c.ready = true;
+}
+
+// Integral blocks of the pair-tensor form (BF16, and nocc > CSF_OMAX): Vt and
+// Ot are the same numbers in the layouts the up contractions read.
 void Handle::build_integrals() {
   IntSet& s = is[0];
   if (s.ready) return;
-  const int o = d.o, v = d.v, naux = d.naux;
+  const int o = d.o, v = d.v;
   const int64_t n1 = d.n1;
   const int64_t nV = (int64_t)v * v * n1, nO = (int64_t)o * o * n1;
-  s.V.alloc(sizeof(double) * nV);
-  s.Vt.alloc(sizeof(double) * nV);
-  s.O.alloc(sizeof(double) * nO);
-  s.Ot.alloc(sizeof(double) * nO);
-  for (int which = 0; which < 2; ++which) {
-    GemmArgs g;
-    const int r = which == 0 ? v : o;
-    g.M = r * r; g.N = (int)n1; g.K = naux;
-    g.A = which == 0 ? (const void*)Bvv.get() : (const void*)Boo.get();
-    g.sam = 1; g.sak = (int64_t)r * r;
-    g.B = Bov.get(); g.sbk = n1; g.sbn = 1;
-    g.map.C = which == 0 ? s.V.get() : s.O.get();
-    g.map.scm = n1; g.map.scn = 1;
-    gemm(g, Prec::F64, gws, st);
+  integral_block(true, s.V);
+  integral_block(false, s.O);
+  if (!csf_form(Prec::F64)) {
+    s.Vt.alloc(sizeof(double) * nV);
+    s.Ot.alloc(sizeof(double) * nO);
+    const double* V = (const double*)s.V.get();
+    for (int c = 0; c < v; ++c)
+      launch_transpose<double, double>(V + (int64_t)c * v * n1, v, n1, (double*)s.Vt.get() + (int64_t)c * n1 * v, st);
+    launch_swap01<double, double>((const double*)s.O.get(), o, o, n1, (double*)s.Ot.get(), st);
   }
-  const double* V = (const double*)s.V.get();
-  for (int c = 0; c < v; ++c)
-    launch_transpose<double, double>(V + (int64_t)c * v * n1, v, n1, (double*)s.Vt.get() + (int64_t)c * n1 * v, st);
-  launch_swap01<double, double>((const double*)s.O.get(), o, o, n1, (double*)s.Ot.get(), st);
+  HIP_CHECK(hipStreamSynchronize(st));
+  s.ready = true;
+}
+
+// Pair-tensor operands of precision p (once).  Where the sigma-vectors of p
+// take the CSF form, only the down operands V and O (the coupled
+// preconditioner's).
+void Handle::ensure_pairs(Prec p) {
+  build_integrals();
+  IntSet& s = is[prec_index(p)];
+  if (s.ready) return;
+  const bool up = !csf_form(p);
+  const IntSet& f = is[0];
+  const int o = d.o, v = d.v;
+  const int64_t n1 = d.n1;
+  const int64_t nV = (int64_t)v * v * n1, nO = (int64_t)o * o * n1;
+  const size_t es = prec_size(p);
+  s.V.alloc(es * nV);
+  if (up) s.Vt.alloc(es * nV);
+  s.O.alloc(es * nO);
+  if (up) s.Ot.alloc(es * nO);
+  const double* V = (const double*)f.V.get();
+  const double* O = (const double*)f.O.get();
+  if (!up) {
+    launch_convert_f32(V, (float*)s.V.get(), nV, st);
+    launch_convert_f32(O, (float*)s.O.get(), nO, st);
+  } else if (p == Prec::F32) {
+    launch_convert_f32(V, (float*)s.V.get(), nV, st);
+    launch_convert_f32(O, (float*)s.O.get(), nO, st);
+    for (int c = 0; c < v; ++c)
+      launch_transpose<double, float>(V + (int64_t)c * v * n1, v, n1, (float*)s.Vt.get() + (int64_t)c * n1 * v, st);
+    launch_swap01<double, float>(O, o, o, n1, (float*)s.Ot.get(), st);
+  } else {
+    launch_convert_bf16(V, (__bf16*)s.V.get(), nV, st);
+    launch_convert_bf16(O, (__bf16*)s.O.get(), nO, st);
+    for (int c = 0; c < v; ++c)
+      launch_transpose<double, __bf16>(V + (int64_t)c * v * n1, v, n1, (__bf16*)s.Vt.get() + (int64_t)c * n1 * v,
+                                       st);
+    launch_swap01<double, __bf16>(O, o, o, n1, (__bf16*)s.Ot.get(), st);
+  }
   HIP_CHECK(hipStreamSynchronize(st));
   s.ready = true;
 }
@@ -147,36 +226,10 @@ void Handle::build_integrals() {
 // or the integral blocks (INT form, rounded from the FP64 ones).
 void Handle::ensure_lowprec(Prec p) {
   if (form == FORM_INT) {
-    build_integrals();
-    IntSet& s = is[prec_index(p)];
-    if (s.ready) return;
-    const IntSet& f = is[0];
-    const int o = d.o, v = d.v;
-    const int64_t n1 = d.n1;
-    const int64_t nV = (int64_t)v * v * n1, nO = (int64_t)o * o * n1;
-    const size_t es = prec_size(p);
-    s.V.alloc(es * nV);
-    s.Vt.alloc(es * nV);
-    s.O.alloc(es * nO);
-    s.Ot.alloc(es * nO);
-    const double* V = (const double*)f.V.get();
-    const double* O = (const double*)f.O.get();
-    if (p == Prec::F32) {
-      launch_convert_f32(V, (float*)s.V.get(), nV, st);
-      launch_convert_f32(O, (float*)s.O.get(), nO, st);
-      for (int c = 0; c < v; ++c)
-        launch_transpose<double, float>(V + (int64_t)c * v * n1, v, n1, (float*)s.Vt.get() + (int64_t)c * n1 * v, st);
-      launch_swap01<double, float>(O, o, o, n1, (float*)s.Ot.get(), st);
-    } else {
-      launch_convert_bf16(V, (__bf16*)s.V.get(), nV, st);
-      launch_convert_bf16(O, (__bf16*)s.O.get(), nO, st);
-      for (int c = 0; c < v; ++c)
-        launch_transpose<double, __bf16>(V + (int64_t)c * v * n1, v, n1, (__bf16*)s.Vt.get() + (int64_t)c * n1 * v,
-                                         st);
-      launch_swap01<double, __bf16>(O, o, o, n1, (__bf16*)s.Ot.get(), st);
-    }
-    HIP_CHECK(hipStreamSynchronize(st));
-    s.ready = true;
+    if (csf_form(p))
+      build_csf(p);
+    else
+      ensure_pairs(p);
     return;
   }
   FactorSet& f = fs[prec_index(p)];
@@ -311,6 +364,7 @@ size_t Handle::sigma_workspace_bytes(int nc, Prec p) const {
 }
 
 bool Handle::lowprec_ready(Prec p) const {
+  if (csf_form(p)) return cs[prec_index(p)].ready;
   return form == FORM_INT ? is[prec_index(p)].ready : (p == Prec::F64 ? fs[0].ready : fs[prec_index(p)].ready);
 }
 
@@ -318,6 +372,16 @@ bool Handle::lowprec_ready(Prec p) const {
 // (256-byte aligned regions) plus at least 32 MiB, or the per-vector
 // workspace if larger, for the GEMM split-K partials.
 int Handle::scratch_chunk(Prec p) const {
+  if (csf_form(p)) {
+    // the partials of the CSF form hardly grow with the vectors; 24 vectors
+    // keep the split-K partials of H11 x1 (about 1 MiB each) within the reserve
+    const size_t reserve = ((size_t)32 << 20) + 3 * 256;
+    for (int nc = 24; nc > 0; --nc) {
+      const CsfBytes b = csf_workspace(dk, nc);
+      if (b.down + b.occ + b.t2 + reserve <= scratch_bytes) return nc;
+    }
+    return 0;
+  }
   const size_t per = sigma_workspace_bytes(1, p) + 6 * 256;
   const size_t reserve = std::max<size_t>((size_t)32 << 20, per);
   if (scratch_bytes < per + reserve) return 0;
@@ -344,7 +408,8 @@ void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nve
   const size_t es = prec_size(p);
   const size_t n1 = d.n1, naux = d.naux;
   const size_t wes = (p == Prec::F64) ? 8 : 4;  // DF W accumulator type
-  int nc_max = std::min(chunk, nvec);
+  // the CSF form needs no n1 x n1 workspace per vector
+  int nc_max = std::min(csf_form(p) ? 64 : chunk, nvec);
   if (scratch) {
     // caller-provided scratch: no allocation; the operands must be resident
     ARG_CHECK(lowprec_ready(p), "the operands of this precision are not resident (create the handle with "
@@ -358,15 +423,22 @@ void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nve
       q += (bytes + 255) / 256 * 256;
       return (void*)r;
     };
-    ws_x1c = carve(n1 * nc_max * es);
-    ws_zg = carve(n1 * n1 * nc_max * es);
-    if (form == FORM_INT) {
-      ws_x1t = carve(n1 * nc_max * es);
+    if (csf_form(p)) {
+      const CsfBytes b = csf_workspace(dk, nc_max);
+      ws_pdown = carve(b.down);
+      ws_pocc = carve(b.occ);
+      ws_pt2 = carve(b.t2);
     } else {
-      ws_yvv = carve(naux * n1 * nc_max * es);
-      ws_yoo = carve(naux * n1 * nc_max * es);
-      ws_wup = carve(naux * n1 * nc_max * wes);
-      ws_wupt = carve(naux * n1 * nc_max * es);
+      ws_x1c = carve(n1 * nc_max * es);
+      ws_zg = carve(n1 * n1 * nc_max * es);
+      if (form == FORM_INT) {
+        ws_x1t = carve(n1 * nc_max * es);
+      } else {
+        ws_yvv = carve(naux * n1 * nc_max * es);
+        ws_yoo = carve(naux * n1 * nc_max * es);
+        ws_wup = carve(naux * n1 * nc_max * wes);
+        ws_wupt = carve(naux * n1 * nc_max * es);
+      }
     }
     ARG_CHECK(q <= scratch + scratch_bytes, "scratch layout exceeds the scratch");
     gws.ext = q;
@@ -375,27 +447,41 @@ void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nve
     ensure_lowprec(p);
     gws.ext = nullptr;
     gws.ext_size = 0;
-    X1c.alloc(n1 * nc_max * es);
-    ZG.alloc(n1 * n1 * nc_max * es);
-    ws_x1c = X1c.get();
-    ws_zg = ZG.get();
-    if (form == FORM_INT) {
-      X1t.alloc(n1 * nc_max * es);
-      ws_x1t = X1t.get();
+    if (csf_form(p)) {
+      const CsfBytes b = csf_workspace(dk, nc_max);
+      Pdown.alloc(b.down);
+      Pocc.alloc(b.occ);
+      Pt2.alloc(b.t2);
+      ws_pdown = Pdown.get();
+      ws_pocc = Pocc.get();
+      ws_pt2 = Pt2.get();
     } else {
-      Yvv.alloc(naux * n1 * nc_max * es);
-      Yoo.alloc(naux * n1 * nc_max * es);
-      Wup.alloc(naux * n1 * nc_max * wes);
-      WupT.alloc(naux * n1 * nc_max * es);
-      ws_yvv = Yvv.get();
-      ws_yoo = Yoo.get();
-      ws_wup = Wup.get();
-      ws_wupt = WupT.get();
+      X1c.alloc(n1 * nc_max * es);
+      ZG.alloc(n1 * n1 * nc_max * es);
+      ws_x1c = X1c.get();
+      ws_zg = ZG.get();
+      if (form == FORM_INT) {
+        X1t.alloc(n1 * nc_max * es);
+        ws_x1t = X1t.get();
+      } else {
+        Yvv.alloc(naux * n1 * nc_max * es);
+        Yoo.alloc(naux * n1 * nc_max * es);
+        Wup.alloc(naux * n1 * nc_max * wes);
+        WupT.alloc(naux * n1 * nc_max * es);
+        ws_yvv = Yvv.get();
+        ws_yoo = Yoo.get();
+        ws_wup = Wup.get();
+        ws_wupt = WupT.get();
+      }
     }
   }
   for (int c0 = 0; c0 < nvec; c0 += nc_max) {
     const int nc = std::min(nc_max, nvec - c0);
-    if (form == FORM_INT)
+    if (csf_form(p) && p == Prec::F64)
+      sigma_csf<double>(X + ldx * c0, ldx, W + ldw * c0, ldw, nc, s);
+    else if (csf_form(p))
+      sigma_csf<float>(X + ldx * c0, ldx, W + ldw * c0, ldw, nc, s);
+    else if (form == FORM_INT)
       sigma_int(X + ldx * c0, ldx, W + ldw * c0, ldw, nc, p, s);
     else
       sigma_df(X + ldx * c0, ldx, W + ldw * c0, ldw, nc, p, s);
@@ -605,6 +691,54 @@ void Handle::sigma_int(const double* Xc, int64_t ldx, double* Wc, int64_t ldw, i
   if (eu.first) HIP_CHECK(hipEventRecord(eu.first, s));
   unpack_chunk(p, ws_zg, Xc, ldx, Wc, ldw, nc, dk, eps.get(), lay, s);
   if (eu.second) HIP_CHECK(hipEventRecord(eu.second, s));
+}
+
+// INT form on the CSF vectors (csf.hip), one chunk of nc vectors:
+//   W1 = H11 x1                                      (FP64)
+//   W2 = D x2 + occupied up, occupied down partials  (FP64, one pass over x2)
+//   W1 += virtual down (precision T) + occupied down
+//   W2 += virtual up (precision T)
+template <class T>
+void Handle::sigma_csf(const double* Xc, int64_t ldx, double* Wc, int64_t ldw, int nc, hipStream_t s) {
+  typedef typename Mma<T>::Acc Acc;
+  const int64_t n1 = d.n1;
+  const T* V = (const T*)cs[std::is_same<T, double>::value ? 0 : 1].V.get();
+  const CsfGeo g = csf_geo<T>(dk, nc, ldx, ldw);
+  const CsfPlan p = csf_plan(dk, nc);
+  const bool down = part != SIGMA_UP, up = part != SIGMA_DOWN;
+  auto span = [&](int cls, double work) -> hipEvent_t {
+    if (!prof_on) return nullptr;
+    hipEvent_t a = prof_event(), b = prof_event();
+    prof.push_back({cls, a, b, work});
+    HIP_CHECK(hipEventRecord(a, s));
+    return b;
+  };
+  auto end = [&](hipEvent_t e) {
+    if (e) HIP_CHECK(hipEventRecord(e, s));
+  };
+  const double flops_v = 2.0 * d.v * (double)n1 * n1 * nc;
+  if (down) {
+    GemmArgs h;
+    h.M = (int)n1; h.N = nc; h.K = (int)n1;
+    h.A = H11.get(); h.sam = n1; h.sak = 1;
+    h.B = Xc; h.sbk = 1; h.sbn = ldx;
+    h.map.C = Wc; h.map.scm = 1; h.map.scn = ldw;
+    gemm(h, Prec::F64, gws, s);
+  }
+  hipEvent_t e = span(2, (double)nc * d.n2 * 8.0 * (up ? 2.0 : 1.0));
+  launch_csf_occ(g, p, Xc, cs_O.get(), eps.get(), Wc, (double*)ws_pocc, (double*)ws_pt2, up, down, s);
+  end(e);
+  if (down) {
+    e = span(0, flops_v);
+    launch_csf_down<T>(g, p, Xc, (const double*)ws_pt2, cs_zeros.get(), V, (Acc*)ws_pdown, s);
+    end(e);
+    launch_csf_reduce<Acc>(g, p, (const Acc*)ws_pdown, (const double*)ws_pocc, Wc, s);
+  }
+  if (up) {
+    e = span(0, flops_v);
+    launch_csf_up<T>(g, p, Xc, cs_zeros.get(), V, Wc, s);
+    end(e);
+  }
 }
 
 // DF form, one chunk of nc vectors (T the GEMM precision p):

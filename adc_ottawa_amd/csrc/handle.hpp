@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "csf.hpp"
 #include "gemm.hpp"
 #include "kernels.hpp"
 
@@ -42,7 +43,19 @@ struct Handle {
     bool ready = false;
   };
   IntSet is[3];
+  // The same form for nocc <= CSF_OMAX in FP64 and FP32: integral operands in
+  // the order of the CSFs (csf.hip), the occupied one in FP64 for both.
+  struct CsfSet {
+    DevBuf<char> V;
+    bool ready = false;
+  };
+  CsfSet cs[2];
+  DevBuf<double> cs_O, cs_zeros;
+  bool csf_form(Prec p) const { return form == FORM_INT && p != Prec::BF16 && d.o <= CSF_OMAX; }
+  void integral_block(bool virt, DevBuf<char>& out);
   void build_integrals();
+  void build_csf(Prec p);
+  void ensure_pairs(Prec p);
   size_t integral_bytes(Prec p) const;
   const void* fBov(Prec p) const;
   const void* fBovT(Prec p) const;
@@ -55,10 +68,11 @@ struct Handle {
   DevBuf<char> Wup;         // W[P][vec][(c,k)] (accumulator type: FP64, or FP32 for FP32/BF16)
   DevBuf<char> WupT;        // W transposed, [(vec,c,k)][P], GEMM precision
   DevBuf<char> ZG;          // Z then G, in the chunk's GEMM precision
+  DevBuf<char> Pdown, Pocc, Pt2;  // 1h1p partials and t2 copy of the CSF form
   // workspaces of the current sigma pass: the buffers above, or regions of
   // a caller's scratch (sigma with `scratch` set allocates nothing)
   void *ws_x1c = nullptr, *ws_x1t = nullptr, *ws_zg = nullptr, *ws_yvv = nullptr, *ws_yoo = nullptr,
-       *ws_wup = nullptr, *ws_wupt = nullptr;
+       *ws_wup = nullptr, *ws_wupt = nullptr, *ws_pdown = nullptr, *ws_pocc = nullptr, *ws_pt2 = nullptr;
   char* scratch = nullptr;
   size_t scratch_bytes = 0;
   bool lowprec_ready(Prec p) const;
@@ -175,6 +189,8 @@ struct Handle {
   void sigma_part(const double* X, int64_t ldx, double* W, int64_t ldw, int nvec, Prec p, int which, hipStream_t s);
   void sigma_df(const double* X, int64_t ldx, double* W, int64_t ldw, int nc, Prec p, hipStream_t s);
   void sigma_int(const double* X, int64_t ldx, double* W, int64_t ldw, int nc, Prec p, hipStream_t s);
+  template <class T>
+  void sigma_csf(const double* X, int64_t ldx, double* W, int64_t ldw, int nc, hipStream_t s);
   // INT form: W1 += C x2 for the nc pair tensors Z (virtual-major layout)
   void int_down(const void* Z, int nc, Prec p, double* W1, int64_t ldw, hipStream_t s);
   size_t sigma_workspace_bytes(int nc, Prec p) const;

@@ -150,6 +150,8 @@ def stream_stats(prof):
     out = {}
     for k in ("csf_to_pair", "pair_to_csf_diag"):
         ms, n, b = prof[k]
+        if n == 0:  # the INT form on CSF vectors has no packing pass
+            continue
         out[k] = {"GBps": round(b / (ms * 1e-3) / 1e9, 1), "frac_of_8TBps": round(b / (ms * 1e-3) / 1e9 / HBM_PEAK, 3),
                   "avg_launch_ms": round(ms / max(n, 1), 4), "bytes_per_launch": b / max(n, 1)}
     return out

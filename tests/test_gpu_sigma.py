@@ -184,3 +184,31 @@ def test_sigma_virtual_200(prec, tol, form):
         W = op.sigma(X, precision=prec)
     ref = df.sigma(X)
     assert np.abs(W - ref).max() < tol * np.abs(ref).max()
+
+
+# INT form on the CSF vectors: nocc at the ends of its range and of the two
+# occupied tile widths (16 | 17), nvirt with pair numbers that fill their last
+# 128-byte chunk or leave one pair in it, with a partial last 16-column block,
+# and with two column splits (v > 208); vector counts that leave partial
+# groups of rows, of vectors per workgroup, and a second pass (> 64)
+CSF_CASES = [(2, 2, 1), (2, 33, 65), (3, 17, 5), (15, 18, 9), (16, 32, 5), (17, 9, 4), (31, 10, 3), (32, 17, 9),
+             (33, 8, 3), (2, 224, 7), (5, 209, 3), (16, 64, 20), (13, 37, 8), (20, 40, 13), (26, 20, 2)]
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
+@pytest.mark.parametrize("o,v,nvec", CSF_CASES)
+def test_sigma_csf_edges(o, v, nvec, prec, tol):
+    print(f"[case] sigma csf edges o={o} v={v} nvec={nvec} {prec}", flush=True)
+    sys = make_system(o, v, 12, seed=o + v)
+    df = dfsigma.DF(sys)
+    X = np.random.default_rng(15).standard_normal((df.n1 + df.D2.size, nvec))
+    ref = df.sigma(X)
+    n1 = df.n1
+    with lib.Operator.from_system(sys, coupling="int") as op:
+        W = op.sigma(X, precision=prec)
+        # each half against its own scale: the 1h1p rows are the larger
+        for rows in (slice(0, n1), slice(n1, None)):
+            assert np.abs(W[rows] - ref[rows]).max() < tol * np.abs(ref[rows]).max()
+        # one vector alone: another launch shape, the same numbers to rounding
+        w = op.sigma(X[:, -1], precision=prec)
+        assert np.abs(w - ref[:, -1]).max() < tol * np.abs(ref[:, -1]).max()
