@@ -9,14 +9,27 @@
 //   G(c,b,k,l) = 1/2 sum_de (cd|be) T(d,e,k,l) + 1/2 sum_mn (km|ln) T(c,b,m,n)
 //              + sum_dm [2 (ck|dm) - (cd|km)] T(d,b,m,l)
 //              - sum_dm [(cl|dm) T(d,b,m,k) + (cd|lm) T(d,b,k,m)],
-// and the block is the CSF projection of G (again with 1/3 on t5).  As
-// matrix products over n1 = o v and v^2 / o^2 pair indices:
+// and the block is the CSF projection of G (again with 1/3 on t5).
+//
+// The ring terms are matrix products over n1 = o v:
 //   G1[(c,k)][(b,l)] = A1 T1,          A1 = 2 (ck|dm) - (cd|km),  T1[(d,m)][(b,l)] = T(d,b,m,l)
 //   G2[(c,l)][(b,k)] = OV T1 + VO T3,  T3[(d,m)][(b,k)] = T(d,b,k,m)
-//   G3[(c,b)][(k,l)] = (VVVV T4 + T4 OOOO) / 2,  T4[(d,e)][(k,l)] = T(d,e,k,l)
-//   G(c,b,k,l) = G1[(c,k),(b,l)] - G2[(c,l),(b,k)] + G3[(c,b),(k,l)].
 // (T1 also serves the (cl|dm) term: T(d,b,m,k) = T(b,d,k,m), the pair
-// symmetry of Z.)  One vector at a time, FP64; the vvvv matrix is v^4 doubles.
+// symmetry of Z).
+//
+// The ladder terms split over the parts of T symmetric (+) and antisymmetric
+// (-) in the virtual pair, which by the pair symmetry are the same in the
+// occupied pair, so that only d <= e, c <= b and k <= l (< for -) remain:
+//   S+-(cb;kl) = G(c,b,k,l) +- G(b,c,k,l)
+//              = 1/2 sum_{d<=e} Kpm(cb;de) Tpm(de;kl) + (oo|oo) likewise,
+//   Kpm(cb;de) = (cd|be) +- (ce|bd).
+// T+ and T- are the CSFs themselves (T+ = sqrt2 x4, -2 x2, x3, -sqrt2 x1 for
+// the pairs of t4, t2, t3, t1; T- = x5 up to a factor), and S+- enter their
+// CSFs directly.  That is 2 (v^2/2)^2 o^2 operations for the (vv|vv) term of a
+// vector instead of the 2 v^4 o^2 of the unsymmetrised matrix (which took
+// 17.6 of the 25.4 ms of 4 vectors at o=14, v=150), and half its storage.
+//
+// FP64.
 #include "handle.hpp"
 
 #include <algorithm>
@@ -63,45 +76,105 @@ __device__ __forceinline__ double ax_t(const double* x, const DimsK& d, int c, i
   return 2.0 * ax_z(x, d, c, b, k, l) - ax_z(x, d, b, c, k, l);
 }
 
-// the three layouts of T for the nb vectors of a chunk (vector j =
-// blockIdx.y), stored transposed -- row (j, column index), contiguous over
-// the contraction index -- so that one matrix product with both operands
-// K-contiguous serves the whole chunk:
-//   T1t[(j,b,l)][(d,m)] = T(d,b,m,l), T3t[(j,b,k)][(d,m)] = T(d,b,k,m),
-//   T4t[(j,k,l)][(d,e)] = T(d,e,k,l), and T4n[(d,e)][(j,k,l)] = T(d,e,k,l)
-//   for the product with the (oo|oo) matrix
-__global__ void ax_layouts_kernel(const double* __restrict__ X, int64_t ldx, DimsK d, int nb,
-                                  double* __restrict__ T1, double* __restrict__ T3, double* __restrict__ T4,
-                                  double* __restrict__ T4n) {
-  const int o = d.o, v = d.v;
+// T1 and T3 for the nb vectors of a chunk (vector j = blockIdx.y), stored
+// transposed -- contiguous over the contraction index:
+//   T1t[j][(b,l)][(d,m)] = T(d,b,m,l), T3t[j][(b,k)][(d,m)] = T(d,b,k,m)
+// (one element per thread, for nocc > 64; launch_pack_t otherwise)
+__global__ void ax_layouts_kernel(const double* __restrict__ X, int64_t ldx, DimsK d, double* __restrict__ T1,
+                                  double* __restrict__ T3) {
+  const int o = d.o;
   const int j = blockIdx.y;
   const double* x = X + ldx * j;
-  const int64_t n1 = d.n1, nn = n1 * n1, oo = (int64_t)o * o;
+  const int64_t n1 = d.n1, nn = n1 * n1;
   for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < nn;
        idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = idx / n1, q = idx - r * n1;
+    const int64_t q = idx / n1, r = idx - q * n1;
     const int dd = (int)(r / o), m = (int)(r - (int64_t)dd * o);
     const int b = (int)(q / o), l = (int)(q - (int64_t)b * o);
-    const int64_t o13 = ((int64_t)j * n1 + q) * n1 + r;
-    T1[o13] = ax_t(x, d, dd, b, m, l);
-    T3[o13] = ax_t(x, d, dd, b, l, m);
-    const int64_t de = idx / oo, kl = idx - de * oo;
-    const int d4 = (int)(de / v), e4 = (int)(de - (int64_t)d4 * v);
-    const int k4 = (int)(kl / o), l4 = (int)(kl - (int64_t)k4 * o);
-    const double t4 = ax_t(x, d, d4, e4, k4, l4);
-    T4[((int64_t)j * oo + kl) * (int64_t)v * v + de] = t4;
-    T4n[(de * nb + j) * oo + kl] = t4;
+    T1[j * nn + idx] = ax_t(x, d, dd, b, m, l);
+    T3[j * nn + idx] = ax_t(x, d, dd, b, l, m);
   }
 }
 
-// G(c,b,k,l) of vector j of a chunk of nb (the column-block layouts above)
-__device__ __forceinline__ double ax_g(const double* G1, const double* G2, const double* G3, const DimsK& d, int nb,
-                                       int j, int c, int b, int k, int l) {
+// Tp[(j, k<=l)][d<=e] and Tm[(j, k<l)][d<e] of the vectors of a chunk, rows of
+// ldp and ldm elements (zeros at their ends): pairs k < l first, then k = l;
+// pairs d < e first, then d = e.
+__global__ void ax_pm_kernel(const double* __restrict__ X, int64_t ldx, int nb, DimsK d, int64_t ldp, int64_t ldm,
+                             double* __restrict__ Tp, double* __restrict__ Tm) {
   const int o = d.o, v = d.v;
-  const int64_t n1 = d.n1, oo = (int64_t)o * o;
-  return G1[(((int64_t)c * o + k) * nb + j) * n1 + (int64_t)b * o + l] -
-         G2[(((int64_t)c * o + l) * nb + j) * n1 + (int64_t)b * o + k] +
-         G3[(((int64_t)c * v + b) * nb + j) * oo + (int64_t)k * o + l];
+  const int64_t so = d.npo + o;
+  const int64_t row = blockIdx.y + (int64_t)gridDim.y * blockIdx.z;
+  if (row >= so * nb) return;
+  const int64_t j = row / so, kl = row - j * so;
+  const double* x = X + ldx * j;
+  double* tp = Tp + row * ldp;
+  double* tm = Tm + (j * d.npo + kl) * ldm;
+  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < ldp; p += (int64_t)gridDim.x * blockDim.x) {
+    double val = 0.0;
+    if (kl < d.npo) {
+      if (p < d.npv) val = AX_SQ2 * x[d.off4 + kl * d.npv + p];
+      else if (p < d.npv + v) val = x[d.off3 + kl * v + p - d.npv];
+      if (p < ldm) tm[p] = p < d.npv ? x[d.off5 + kl * d.npv + p] : 0.0;
+    } else {
+      const int64_t k = kl - d.npo;
+      if (p < d.npv) val = -2.0 * x[d.off2 + p * o + k];
+      else if (p < d.npv + v) val = -AX_SQ2 * x[d.off1 + k * v + p - d.npv];
+    }
+    tp[p] = val;
+  }
+}
+
+// Kp[(c<=b)][(d<=e)], Km[(c<b)][(d<e)] from I[c][d][b][e] = (cd|be)
+__global__ void ax_kpm_kernel(const double* __restrict__ I, DimsK d, int64_t ldp, int64_t ldm,
+                              double* __restrict__ Kp, double* __restrict__ Km) {
+  const int v = d.v;
+  const int64_t r = blockIdx.y + (int64_t)gridDim.y * blockIdx.z;
+  if (r >= d.npv + v) return;
+  int c, b;
+  if (r < d.npv) ax_unpair(r, v, c, b);
+  else c = b = (int)(r - d.npv);
+  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < ldp; p += (int64_t)gridDim.x * blockDim.x) {
+    double kp = 0.0, km = 0.0;
+    if (p < d.npv + v) {
+      int dd, e;
+      if (p < d.npv) ax_unpair(p, v, dd, e);
+      else dd = e = (int)(p - d.npv);
+      const double g1 = I[(((int64_t)c * v + dd) * v + b) * v + e], g2 = I[(((int64_t)c * v + e) * v + b) * v + dd];
+      kp = g1 + g2;
+      km = g1 - g2;
+    }
+    Kp[r * ldp + p] = kp;
+    if (r < d.npv && p < ldm) Km[r * ldm + p] = p < d.npv ? km : 0.0;
+  }
+}
+
+// Op[(k<=l)][(m<=n)] = (km|ln) + (kn|lm) (m < n), (km|lm) (m = n); Om with a
+// minus sign and no equal pairs.  oooo[(m,n)][(k,l)] = (km|ln).
+__global__ void ax_opm_kernel(const double* __restrict__ oooo, DimsK d, double* __restrict__ Op,
+                              double* __restrict__ Om) {
+  const int o = d.o;
+  const int64_t so = d.npo + o;
+  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < so * so;
+       idx += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = idx / so, q = idx - r * so;
+    int k, l, m, n;
+    if (r < d.npo) ax_unpair(r, o, k, l);
+    else k = l = (int)(r - d.npo);
+    if (q < d.npo) ax_unpair(q, o, m, n);
+    else m = n = (int)(q - d.npo);
+    const double g1 = oooo[(((int64_t)m * o + n) * o + k) * o + l], g2 = oooo[(((int64_t)n * o + m) * o + k) * o + l];
+    Op[idx] = m == n ? g1 : g1 + g2;
+    if (r < d.npo && q < d.npo) Om[r * d.npo + q] = g1 - g2;
+  }
+}
+
+// ring part of G(c,b,k,l) of vector j
+__device__ __forceinline__ double ax_g(const double* G1, const double* G2, const DimsK& d, int j, int c, int b, int k,
+                                       int l) {
+  const int o = d.o;
+  const int64_t n1 = d.n1, base = (int64_t)j * n1 * n1;
+  return G1[base + ((int64_t)c * o + k) * n1 + (int64_t)b * o + l] -
+         G2[base + ((int64_t)c * o + l) * n1 + (int64_t)b * o + k];
 }
 
 // 2h2p configuration J (0-based within the 2h2p part) -> type 1..5 and (a, b, k, l)
@@ -133,11 +206,10 @@ __device__ __forceinline__ int ax_decode(int64_t J, const DimsK& d, int& a, int&
   return t;
 }
 
-// w[off1 + J] += (M22 x)_J from G (the CSF projection, 1/3 on t5), vector
-// j = blockIdx.y of the chunk
-__global__ void ax_project_kernel(const double* __restrict__ G1, const double* __restrict__ G2,
-                                  const double* __restrict__ G3, DimsK d, int nb, double* __restrict__ W,
-                                  int64_t ldw) {
+// w[off1 + J] += (M22 x)_J of the ring terms (the CSF projection of G, 1/3 on
+// t5), vector j = blockIdx.y (for nocc > 64; launch_unpack_g otherwise)
+__global__ void ax_project_kernel(const double* __restrict__ G1, const double* __restrict__ G2, DimsK d,
+                                  double* __restrict__ W, int64_t ldw) {
   const int64_t n2 = d.ndim - d.n1;
   const int j = blockIdx.y;
   double* w = W + ldw * j;
@@ -146,17 +218,47 @@ __global__ void ax_project_kernel(const double* __restrict__ G1, const double* _
     const int t = ax_decode(J, d, a, b, k, l);
     double val;
     if (t == 1) {
-      val = -AX_SQ2 * ax_g(G1, G2, G3, d, nb, j, a, a, k, k);
+      val = -AX_SQ2 * ax_g(G1, G2, d, j, a, a, k, k);
     } else if (t == 2) {
-      val = -(ax_g(G1, G2, G3, d, nb, j, a, b, k, k) + ax_g(G1, G2, G3, d, nb, j, b, a, k, k));
+      val = -(ax_g(G1, G2, d, j, a, b, k, k) + ax_g(G1, G2, d, j, b, a, k, k));
     } else if (t == 3) {
-      val = ax_g(G1, G2, G3, d, nb, j, a, a, k, l) + ax_g(G1, G2, G3, d, nb, j, a, a, l, k);
+      val = ax_g(G1, G2, d, j, a, a, k, l) + ax_g(G1, G2, d, j, a, a, l, k);
     } else {
-      const double g1 = ax_g(G1, G2, G3, d, nb, j, a, b, k, l), g2 = ax_g(G1, G2, G3, d, nb, j, b, a, k, l);
-      const double g3 = ax_g(G1, G2, G3, d, nb, j, a, b, l, k), g4 = ax_g(G1, G2, G3, d, nb, j, b, a, l, k);
+      const double g1 = ax_g(G1, G2, d, j, a, b, k, l), g2 = ax_g(G1, G2, d, j, b, a, k, l);
+      const double g3 = ax_g(G1, G2, d, j, a, b, l, k), g4 = ax_g(G1, G2, d, j, b, a, l, k);
       val = (t == 4) ? AX_ISQ2 * (g1 + g2 + g3 + g4) : (AX_SQ32 / 3.0) * (g1 - g2 - g3 + g4);
     }
     w[d.off1 + J] += val;
+  }
+}
+
+// the ladder terms: w4 += sqrt2 S+, w3 += S+, w2 -= S+, w1 -= S+ / sqrt2, w5 +=
+// S- (already in units of x5), rows as in ax_pm_kernel
+__global__ void ax_ladder_kernel(const double* __restrict__ Sp, const double* __restrict__ Sm, int nb, DimsK d,
+                                 int64_t ldp, int64_t ldm, double* __restrict__ W, int64_t ldw) {
+  const int o = d.o, v = d.v;
+  const int64_t so = d.npo + o;
+  const int64_t row = blockIdx.y + (int64_t)gridDim.y * blockIdx.z;
+  if (row >= so * nb) return;
+  const int64_t j = row / so, kl = row - j * so;
+  double* w = W + ldw * j;
+  const double* sp = Sp + row * ldp;
+  const double* sm = Sm + (j * d.npo + kl) * ldm;
+  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < d.npv + v;
+       p += (int64_t)gridDim.x * blockDim.x) {
+    const double s = sp[p];
+    if (kl < d.npo) {
+      if (p < d.npv) {
+        w[d.off4 + kl * d.npv + p] += AX_SQ2 * s;
+        w[d.off5 + kl * d.npv + p] += sm[p];
+      } else {
+        w[d.off3 + kl * v + p - d.npv] += s;
+      }
+    } else {
+      const int64_t k = kl - d.npo;
+      if (p < d.npv) w[d.off2 + p * o + k] -= s;
+      else w[d.off1 + k * v + p - d.npv] -= AX_ISQ2 * s;
+    }
   }
 }
 
@@ -169,7 +271,7 @@ __device__ double ax_kpp(const AxMats& M, const DimsK& d, int c, int b, int k, i
   const int o = d.o, v = d.v;
   const int64_t n1 = d.n1;
   double r = 0.0;
-  if (k == m && l == n) r += 0.5 * M.vvvv[(((int64_t)c * v + b) * v + dd) * v + e];
+  if (k == m && l == n) r += 0.5 * M.vvvv[(((int64_t)c * v + dd) * v + b) * v + e];
   if (c == dd && b == e) r += 0.5 * M.oooo[(((int64_t)m * o + n) * o + k) * o + l];
   if (b == e) {
     if (n == l) r += M.a1[((int64_t)c * o + k) * n1 + (int64_t)dd * o + m];
@@ -250,6 +352,9 @@ __global__ void ax_add_kernel(int64_t n, double s, const double* __restrict__ x,
     y[i] += s * x[i];
 }
 
+// rows padded to whole K tiles of the products
+inline int64_t ax_ld(int64_t n) { return (n + 15) / 16 * 16; }
+
 // C (M x N, ldc) = alpha A (M x K, lda) Bt^T + beta C with Bt N x K (ldbt): both
 // operands contiguous along K (the vector loads and the wide tiles)
 void ax_gemm_bt(Handle& H, int M, int N, int K, const double* A, int64_t lda, const double* Bt, int64_t ldbt,
@@ -303,22 +408,27 @@ void Handle::enable_adcx(bool on) {
     hipLaunchKernelGGL(ax_axpby_kernel, dim3(grid_for(n1 * n1)), dim3(256), 0, st, n1 * n1, 2.0, ax_ov.get(), -1.0,
                        ax_vo.get(), ax_a1.get());
     HIP_CHECK(hipGetLastError());
-    // (cd|be) as [(c,b)][(d,e)] and (km|ln) as [(m,n)][(k,l)]
-    ax_vvvv.alloc((size_t)vv * vv);
+    // I[(c,d)][(b,e)] = (cd|be): its symmetric and antisymmetric parts and,
+    // with it, the diagonal of the block
+    DevBuf<double> I;
+    I.alloc((size_t)vv * vv);
     {
-      DevBuf<double> W;  // [(c,d)][(b,e)]
-      W.alloc((size_t)vv * vv);
       GemmArgs g;
       g.M = (int)vv; g.N = (int)vv; g.K = naux;
       g.A = Bvv.get(); g.sam = 1; g.sak = vv;
       g.B = Bvv.get(); g.sbk = vv; g.sbn = 1;
-      g.map.C = W.get(); g.map.scm = vv; g.map.scn = 1;
+      g.map.C = I.get(); g.map.scm = vv; g.map.scn = 1;
       gemm(g, Prec::F64, gws, st);
-      hipLaunchKernelGGL(ax_swap_mid_kernel, dim3(grid_for(vv * vv)), dim3(256), 0, st, W.get(), (int64_t)v,
-                         (int64_t)v, (int64_t)v, (int64_t)v, ax_vvvv.get());
-      HIP_CHECK(hipGetLastError());
-      HIP_CHECK(hipStreamSynchronize(st));
     }
+    const int64_t sv = d.npv + v, ldp = ax_ld(sv), ldm = ax_ld(d.npv);
+    ax_kp.alloc((size_t)sv * ldp);
+    ax_km.alloc((size_t)d.npv * ldm);
+    hipLaunchKernelGGL(ax_kpm_kernel, dim3((unsigned)std::min<int64_t>((ldp + 255) / 256, 64), 4096,
+                                           (unsigned)((sv + 4095) / 4096)),
+                       dim3(256), 0, st, I.get(), dk, ldp, ldm, ax_kp.get(), ax_km.get());
+    HIP_CHECK(hipGetLastError());
+    // (km|ln) as [(m,n)][(k,l)]
+    DevBuf<double> ax_oooo;
     ax_oooo.alloc((size_t)oo * oo);
     {
       DevBuf<double> Q;  // [(k,m)][(l,n)] = (km|ln)
@@ -340,8 +450,14 @@ void Handle::enable_adcx(bool on) {
       launch_transpose<double, double>(R.get(), oo, oo, ax_oooo.get(), st);
       HIP_CHECK(hipStreamSynchronize(st));
     }
+    const int64_t so = d.npo + o;
+    ax_op.alloc((size_t)so * so);
+    ax_om.alloc((size_t)d.npo * d.npo);
+    hipLaunchKernelGGL(ax_opm_kernel, dim3(grid_for(so * so)), dim3(256), 0, st, ax_oooo.get(), dk, ax_op.get(),
+                       ax_om.get());
+    HIP_CHECK(hipGetLastError());
     ax_d2.alloc((size_t)n2);
-    AxMats M{ax_vvvv.get(), ax_oooo.get(), ax_ov.get(), ax_vo.get(), ax_a1.get()};
+    AxMats M{I.get(), ax_oooo.get(), ax_ov.get(), ax_vo.get(), ax_a1.get()};
     hipLaunchKernelGGL(ax_diag_kernel, dim3(grid_for(n2)), dim3(256), 0, st, M, dk, ax_d2.get());
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(st));
@@ -357,40 +473,69 @@ void Handle::enable_adcx(bool on) {
 void Handle::adcx_apply(const double* X, int64_t ldx, double* W, int64_t ldw, int nvec, hipStream_t s) {
   ARG_CHECK(!scratch, "the no-allocation sigma-vector does not include the ADC(2)-x block");
   const int o = d.o, v = d.v;
-  const int64_t n1 = d.n1, nn = n1 * n1, vv = (int64_t)v * v, oo = (int64_t)o * o;
-  // vectors per chunk: seven n1 x n1 arrays per vector within about 4 GB
-  const int64_t per_vec = 7 * nn * (int64_t)sizeof(double);
+  const int64_t n1 = d.n1, nn = n1 * n1;
+  const int64_t sv = d.npv + v, so = d.npo + o, ldp = ax_ld(sv), ldm = ax_ld(d.npv);
+  // vectors per chunk: about six n1 x n1 arrays per vector within about 4 GB
+  const int64_t per_vec = 6 * nn * (int64_t)sizeof(double);
   const int cap = (int)std::max<int64_t>(1, std::min<int64_t>(16, ((int64_t)4 << 30) / per_vec));
   const int nbmax = std::min(nvec, cap);
   ax_t1.alloc((size_t)nbmax * nn);
   ax_t3.alloc((size_t)nbmax * nn);
-  ax_t4.alloc((size_t)nbmax * nn);
-  ax_t4n.alloc((size_t)nbmax * nn);
   ax_g1.alloc((size_t)nbmax * nn);
   ax_g2.alloc((size_t)nbmax * nn);
-  ax_g3.alloc((size_t)nbmax * nn);
+  ax_tp.alloc((size_t)nbmax * so * ldp);
+  ax_tm.alloc((size_t)nbmax * d.npo * ldm);
+  ax_sp.alloc((size_t)nbmax * so * ldp);
+  ax_sm.alloc((size_t)nbmax * d.npo * ldm);
+  const PairLayout lay = pair_layout_vec_major(dk);
   for (int j0 = 0; j0 < nvec; j0 += nbmax) {
     const int nb = std::min(nbmax, nvec - j0);
-    const int64_t w1 = (int64_t)nb * n1, w4 = (int64_t)nb * oo;  // row lengths of the chunk layouts
-    hipLaunchKernelGGL(ax_layouts_kernel, dim3(grid_for(nn), nb), dim3(256), 0, s, X + ldx * j0, ldx, dk, nb,
-                       ax_t1.get(), ax_t3.get(), ax_t4.get(), ax_t4n.get());
-    HIP_CHECK(hipGetLastError());
-    ax_gemm_bt(*this, (int)n1, (int)w1, (int)n1, ax_a1.get(), n1, ax_t1.get(), n1, ax_g1.get(), w1, 1.0, 0.0, s);
-    ax_gemm_bt(*this, (int)n1, (int)w1, (int)n1, ax_ov.get(), n1, ax_t1.get(), n1, ax_g2.get(), w1, 1.0, 0.0, s);
-    ax_gemm_bt(*this, (int)n1, (int)w1, (int)n1, ax_vo.get(), n1, ax_t3.get(), n1, ax_g2.get(), w1, 1.0, 1.0, s);
-    ax_gemm_bt(*this, (int)vv, (int)w4, (int)vv, ax_vvvv.get(), vv, ax_t4.get(), vv, ax_g3.get(), w4, 0.5, 0.0, s);
-    {  // G3 += T4 OOOO / 2 for each vector of the chunk (batch = vector); OOOO is symmetric
-       // ((km|ln) = (mk|nl)), so B(mn, kl) = OOOO[(k,l)][(m,n)] is contiguous along K too
-      GemmArgs g;
-      g.M = (int)vv; g.N = (int)oo; g.K = (int)oo; g.batch = nb;
-      g.A = ax_t4n.get(); g.sam = w4; g.sak = 1; g.sab = oo;
-      g.B = ax_oooo.get(); g.sbk = 1; g.sbn = oo; g.sbb = 0;
-      g.map.C = ax_g3.get(); g.map.scm = w4; g.map.scn = 1; g.map.scb = oo;
-      g.map.alpha = 0.5; g.map.beta = 1.0;
-      gemm(g, Prec::F64, gws, s);
+    const double* x = X + ldx * j0;
+    double* w = W + ldw * j0;
+    if (!launch_pack_t(x, ldx, nb, dk, ax_t1.get(), ax_t3.get(), lay, s)) {
+      hipLaunchKernelGGL(ax_layouts_kernel, dim3(grid_for(nn), nb), dim3(256), 0, s, x, ldx, dk, ax_t1.get(),
+                         ax_t3.get());
+      HIP_CHECK(hipGetLastError());
     }
-    hipLaunchKernelGGL(ax_project_kernel, dim3(grid_for(d.ndim - n1), nb), dim3(256), 0, s, ax_g1.get(),
-                       ax_g2.get(), ax_g3.get(), dk, nb, W + ldw * j0, ldw);
+    auto ring = [&](const double* A, const double* T, double* G, double beta) {
+      GemmArgs g;
+      g.M = (int)n1; g.N = (int)n1; g.K = (int)n1; g.batch = nb;
+      g.A = A; g.sam = n1; g.sak = 1; g.sab = 0;
+      g.B = T; g.sbk = 1; g.sbn = n1; g.sbb = nn;
+      g.map.C = G; g.map.scm = n1; g.map.scn = 1; g.map.scb = nn; g.map.beta = beta;
+      gemm(g, Prec::F64, gws, s);
+    };
+    ring(ax_a1.get(), ax_t1.get(), ax_g1.get(), 0.0);
+    ring(ax_ov.get(), ax_t1.get(), ax_g2.get(), 0.0);
+    ring(ax_vo.get(), ax_t3.get(), ax_g2.get(), 1.0);
+    if (!launch_unpack_g(ax_g1.get(), ax_g2.get(), w, ldw, nb, dk, lay, s)) {
+      hipLaunchKernelGGL(ax_project_kernel, dim3(grid_for(d.ndim - n1), nb), dim3(256), 0, s, ax_g1.get(),
+                         ax_g2.get(), dk, w, ldw);
+      HIP_CHECK(hipGetLastError());
+    }
+    // ladder: rows (vector, kl), columns cb; T and K contiguous along de
+    const unsigned ry = (unsigned)std::min<int64_t>(nb * so, 32768);
+    const dim3 rows((unsigned)std::min<int64_t>((ldp + 255) / 256, 64), ry, (unsigned)((nb * so + ry - 1) / ry));
+    hipLaunchKernelGGL(ax_pm_kernel, rows, dim3(256), 0, s, x, ldx, nb, dk, ldp, ldm, ax_tp.get(), ax_tm.get());
+    HIP_CHECK(hipGetLastError());
+    ax_gemm_bt(*this, (int)(nb * so), (int)sv, (int)ldp, ax_tp.get(), ldp, ax_kp.get(), ldp, ax_sp.get(), ldp, 0.5,
+               0.0, s);
+    ax_gemm_bt(*this, (int)(nb * d.npo), (int)d.npv, (int)ldm, ax_tm.get(), ldm, ax_km.get(), ldm, ax_sm.get(), ldm,
+               1.0, 0.0, s);
+    auto occ = [&](const double* O, int64_t n, const double* T, int64_t ld, double* S, int64_t col0, int64_t ncol,
+                   double alpha) {  // S[(j,kl)][cb] += alpha O[kl][mn] T[(j,mn)][cb]
+      if (ncol <= 0) return;
+      GemmArgs g;
+      g.M = (int)n; g.N = (int)ncol; g.K = (int)n; g.batch = nb;
+      g.A = O; g.sam = n; g.sak = 1; g.sab = 0;
+      g.B = T + col0; g.sbk = ld; g.sbn = 1; g.sbb = n * ld;
+      g.map.C = S + col0; g.map.scm = ld; g.map.scn = 1; g.map.scb = n * ld; g.map.alpha = alpha; g.map.beta = 1.0;
+      gemm(g, Prec::F64, gws, s);
+    };
+    occ(ax_op.get(), so, ax_tp.get(), ldp, ax_sp.get(), 0, d.npv, 0.5);
+    occ(ax_op.get(), so, ax_tp.get(), ldp, ax_sp.get(), d.npv, v, 1.0);  // (T+ of c = b is not doubled)
+    occ(ax_om.get(), d.npo, ax_tm.get(), ldm, ax_sm.get(), 0, d.npv, 1.0);
+    hipLaunchKernelGGL(ax_ladder_kernel, rows, dim3(256), 0, s, ax_sp.get(), ax_sm.get(), nb, dk, ldp, ldm, w, ldw);
     HIP_CHECK(hipGetLastError());
   }
 }

@@ -129,14 +129,13 @@ struct Handle {
   void sigma_view(const double* X, int64_t ldx, double* W, int64_t ldw, int nvec, Prec p, hipStream_t s);
 
   // ADC(2)-x: the first-order 2h2p-2h2p block added to the sigma-vector
-  // (FP64, one vector at a time) and its diagonal to hii.  Integral matrices
-  // (built on enable): ax_vvvv [(c,b)][(d,e)] = (cd|be), ax_oooo [(m,n)][(k,l)]
-  // = (km|ln), ax_ov [(c,k)][(d,m)] = (ck|dm), ax_vo [(c,k)][(d,m)] = (cd|km),
-  // ax_a1 = 2 ax_ov - ax_vo; per-vector layouts of T = 2Z - XZ and of the
-  // three partial results (adcx.hip).
+  // (FP64) and its diagonal to hii.  Integral matrices (built on enable):
+  // ax_kp, ax_km [(c<=b)][(d<=e)] = (cd|be) +- (ce|bd), ax_op, ax_om the same of
+  // (oo|oo), ax_ov [(c,k)][(d,m)] = (ck|dm), ax_vo [(c,k)][(d,m)] = (cd|km), ax_a1
+  // = 2 ax_ov - ax_vo; per-chunk layouts of T and partial results (adcx.hip).
   bool adcx = false;
-  DevBuf<double> ax_vvvv, ax_oooo, ax_ov, ax_vo, ax_a1, ax_d2;
-  DevBuf<double> ax_t1, ax_t3, ax_t4, ax_t4n, ax_g1, ax_g2, ax_g3;
+  DevBuf<double> ax_kp, ax_km, ax_op, ax_om, ax_ov, ax_vo, ax_a1, ax_d2;
+  DevBuf<double> ax_t1, ax_t3, ax_g1, ax_g2, ax_tp, ax_tm, ax_sp, ax_sm;
   void enable_adcx(bool on);
   void adcx_apply(const double* X, int64_t ldx, double* W, int64_t ldw, int nvec, hipStream_t s);
 

@@ -73,6 +73,13 @@ void launch_pack_tiled(const double* X, int64_t ldx, int nvec, const DimsK& d, T
 template <class T>
 void launch_unpack_tiled(const T* G, const double* X, int64_t ldx, double* W, int64_t ldw, int nvec, const DimsK& d,
                          const double* eps, const PairLayout& lay, hipStream_t st);
+// ADC(2)-x (adcx.hip): T1[(a,k)][(b,l)] = T(a,b,k,l) and T3 = T(a,b,l,k) of T = 2Z - XZ,
+// and W += the projection of G1(c,b,k,l) - G2(c,b,l,k); both false (nothing
+// launched) for nocc > 64.
+bool launch_pack_t(const double* X, int64_t ldx, int nvec, const DimsK& d, double* T1, double* T3,
+                   const PairLayout& lay, hipStream_t st);
+bool launch_unpack_g(const double* G1, const double* G2, double* W, int64_t ldw, int nvec, const DimsK& d,
+                     const PairLayout& lay, hipStream_t st);
 // hii[j] for the whole vector: diag(H11) and the 2h2p orbital-energy sums
 void launch_diagonal(const double* H11, const double* eps, const DimsK& d, double* hii, hipStream_t st);
 

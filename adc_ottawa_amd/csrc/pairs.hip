@@ -36,9 +36,12 @@ __device__ __forceinline__ double dbl(T x) { return (double)x; }
 template <>
 __device__ __forceinline__ double dbl<__bf16>(__bf16 x) { return (double)(float)x; }
 
-template <class T>
+// TT (ADC(2)-x): writes T = 2Z - XZ of the amplitudes with t5 weighted by 1/3
+// to Z, and T(a,b,l,k) at (a,b,k,l) to Z3.
+template <class T, bool TT = false>
 __global__ void __launch_bounds__(PT) pack_tiled_kernel(const double* __restrict__ X, int64_t ldx, DimsK d,
-                                                         T* __restrict__ Z, PairLayout lay, int BB) {
+                                                         T* __restrict__ Z, PairLayout lay, int BB,
+                                                         T* __restrict__ Z3 = nullptr) {
   extern __shared__ double sm[];
   const int o = d.o, v = d.v, tid = threadIdx.x;
   const int a = blockIdx.x;
@@ -62,6 +65,7 @@ __global__ void __launch_bounds__(PT) pack_tiled_kernel(const double* __restrict
       if (k == l) val = -SQRT2 * x[d.off1 + (int64_t)k * v + a];
       else val = x[d.off3 + pidx(min(k, l), max(k, l), o) * v + a];
       z[(int64_t)a * sc + (int64_t)k * n1 + (int64_t)a * o + l] = cvt<T>(val);
+      if (TT) Z3[vec * lay.sv + (int64_t)a * sc + (int64_t)k * n1 + (int64_t)a * o + l] = cvt<T>(val);
     }
   }
   if (b0 < v) {
@@ -71,7 +75,7 @@ __global__ void __launch_bounds__(PT) pack_tiled_kernel(const double* __restrict
       const int q = t / nb, bb = t - q * nb;
       const int64_t J = (int64_t)q * npv + p0 + bb;
       xs4[q * BP + bb] = INV_SQRT2 * x[d.off4 + J];
-      xs5[q * BP + bb] = SQRT3_2 * x[d.off5 + J];
+      xs5[q * BP + bb] = (TT ? SQRT3_2 / 3.0 : SQRT3_2) * x[d.off5 + J];
     }
     for (int t = tid; t < nb * o; t += PT) {
       const int bb = t / o, k = t - bb * o;
@@ -97,18 +101,28 @@ __global__ void __launch_bounds__(PT) pack_tiled_kernel(const double* __restrict
           vab = p4 + s_ab * p5;
           vba = p4 - s_ab * p5;
         }
-        zab[(int64_t)bb * o] = cvt<T>(vab);
-        zba[(int64_t)bb * sc] = cvt<T>(vba);
+        if (TT) {
+          const double tab = 2.0 * vab - vba, tba = 2.0 * vba - vab;
+          zab[(int64_t)bb * o] = cvt<T>(tab);
+          zba[(int64_t)bb * sc] = cvt<T>(tba);
+          Z3[(zab - Z) + (int64_t)bb * o] = cvt<T>(tba);
+          Z3[(zba - Z) + (int64_t)bb * sc] = cvt<T>(tab);
+        } else {
+          zab[(int64_t)bb * o] = cvt<T>(vab);
+          zba[(int64_t)bb * sc] = cvt<T>(vba);
+        }
       }
     }
   }
 }
 
-template <class T>
+// TT (ADC(2)-x ring terms): W += the projection of G(c,b,k,l) - G2(c,b,l,k), 1/3
+// on t5, instead of W = the projection + D x.
+template <class T, bool TT = false>
 __global__ void __launch_bounds__(PT) unpack_tiled_kernel(const T* __restrict__ G, const double* __restrict__ X,
                                                            int64_t ldx, double* __restrict__ W, int64_t ldw, DimsK d,
                                                            const double* __restrict__ eps, PairLayout lay, int BB,
-                                                           int op) {
+                                                           int op, const T* __restrict__ G2 = nullptr) {
   extern __shared__ double sm[];
   const int o = d.o, v = d.v, tid = threadIdx.x;
   const int a = blockIdx.x;
@@ -126,14 +140,20 @@ __global__ void __launch_bounds__(PT) unpack_tiled_kernel(const T* __restrict__ 
   // differ across b)
   double* tab = sm;            // [BB][o*o + 1]  G[(a,k),(b,l)]
   double* tba = sm + BB * op;  // [BB][o*o + 1]  G[(b,k),(a,l)]
-  const double ea = eps[o + a];
+  const double ea = TT ? 0.0 : eps[o + a];
+  const T* g2v = TT ? G2 + vec * lay.sv : nullptr;
   // diagonal tile b = a: t1 and t3 (first chunk)
   if (chunk == 0) {
-    for (int t = tid; t < oo; t += PT) tab[t] = dbl(g[(int64_t)a * sc + (int64_t)(t / o) * n1 + (int64_t)a * o + t % o]);
+    for (int t = tid; t < oo; t += PT) {
+      const int64_t r = (int64_t)a * sc + (int64_t)a * o;
+      tab[t] = dbl(g[r + (int64_t)(t / o) * n1 + t % o]);
+      if (TT) tab[t] -= dbl(g2v[r + (int64_t)(t % o) * n1 + t / o]);
+    }
     __syncthreads();
     for (int k = tid; k < o; k += PT) {
       const int64_t J = d.off1 + (int64_t)k * v + a;
-      w[J] = -SQRT2 * tab[k * o + k] + (2.0 * ea - 2.0 * eps[k]) * x[J];
+      if (TT) w[J] += -SQRT2 * tab[k * o + k];
+      else w[J] = -SQRT2 * tab[k * o + k] + (2.0 * ea - 2.0 * eps[k]) * x[J];
     }
     for (int q = tid; q < npo; q += PT) {
       // decode q -> (k, l) by walking the rows (npo is small)
@@ -145,7 +165,8 @@ __global__ void __launch_bounds__(PT) unpack_tiled_kernel(const T* __restrict__ 
       }
       const int l = (int)(q - base) + k + 1;
       const int64_t J = d.off3 + (int64_t)q * v + a;
-      w[J] = tab[k * o + l] + tab[l * o + k] + (2.0 * ea - eps[k] - eps[l]) * x[J];
+      if (TT) w[J] += tab[k * o + l] + tab[l * o + k];
+      else w[J] = tab[k * o + l] + tab[l * o + k] + (2.0 * ea - eps[k] - eps[l]) * x[J];
     }
   }
   if (b0 < v) {
@@ -162,10 +183,26 @@ __global__ void __launch_bounds__(PT) unpack_tiled_kernel(const T* __restrict__ 
       }
     }
     __syncthreads();
+    if (TT) {  // G2 with its occupied indices turned
+      for (int kl = tid; kl < oo; kl += PT) {
+        const int k = kl / o, l = kl - k * o;
+        const T* gab = g2v + (int64_t)a * sc + (int64_t)k * n1 + (int64_t)b0 * o + l;
+        const T* gba = g2v + (int64_t)b0 * sc + (int64_t)k * n1 + (int64_t)a * o + l;
+        for (int bb = 0; bb < nb; ++bb) {
+          tab[bb * op + l * o + k] -= dbl(gab[(int64_t)bb * o]);
+          tba[bb * op + l * o + k] -= dbl(gba[(int64_t)bb * sc]);
+        }
+      }
+      __syncthreads();
+    }
     // t2 (a<b, k=l): contiguous over (b, k)
     for (int t = tid; t < nb * o; t += PT) {
       const int bb = t / o, k = t - bb * o;
       const int64_t J = d.off2 + (p0 + bb) * o + k;
+      if (TT) {
+        w[J] -= tab[bb * op + k * o + k] + tba[bb * op + k * o + k];
+        continue;
+      }
       const double D = ea + eps[o + b0 + bb] - 2.0 * eps[k];
       w[J] = -(tab[bb * op + k * o + k] + tba[bb * op + k * o + k]) + D * x[J];
     }
@@ -183,8 +220,13 @@ __global__ void __launch_bounds__(PT) unpack_tiled_kernel(const T* __restrict__ 
       const double* A = tab + bb * op;
       const double* Bt = tba + bb * op;
       const double g1 = A[k * o + l], g3 = A[l * o + k], g2 = Bt[k * o + l], g4 = Bt[l * o + k];
-      const double D = ea + eps[o + b0 + bb] - eps[k] - eps[l];
       const int64_t J = (int64_t)q * npv + p0 + bb;
+      if (TT) {
+        w[d.off4 + J] += INV_SQRT2 * (g1 + g2 + g3 + g4);
+        w[d.off5 + J] += (SQRT3_2 / 3.0) * (g1 - g2 - g3 + g4);
+        continue;
+      }
+      const double D = ea + eps[o + b0 + bb] - eps[k] - eps[l];
       w[d.off4 + J] = INV_SQRT2 * (g1 + g2 + g3 + g4) + D * x[d.off4 + J];
       w[d.off5 + J] = SQRT3_2 * (g1 - g2 - g3 + g4) + D * x[d.off5 + J];
     }
@@ -225,6 +267,32 @@ void launch_unpack_tiled(const T* G, const double* X, int64_t ldx, double* W, in
   hipLaunchKernelGGL((unpack_tiled_kernel<T>), dim3(d.v, std::max(chunks, 1), nvec), dim3(PT), lds, st, G, X, ldx, W,
                      ldw, d, eps, lay, BB, op);
   HIP_CHECK(hipGetLastError());
+}
+
+bool launch_pack_t(const double* X, int64_t ldx, int nvec, const DimsK& d, double* T1, double* T3,
+                   const PairLayout& lay, hipStream_t st) {
+  if (d.o > 64) return false;
+  const int BB = pack_chunk(d);
+  const size_t lds = sizeof(double) * ((size_t)(BB + 1) * 2 * d.npo + (size_t)BB * d.o);
+  const int chunks = (d.v - 1 + BB - 1) / BB;
+  hipLaunchKernelGGL((pack_tiled_kernel<double, true>), dim3(d.v, std::max(chunks, 1), nvec), dim3(PT), lds, st, X, ldx,
+                     d, T1, lay, BB, T3);
+  HIP_CHECK(hipGetLastError());
+  return true;
+}
+
+bool launch_unpack_g(const double* G1, const double* G2, double* W, int64_t ldw, int nvec, const DimsK& d,
+                     const PairLayout& lay, hipStream_t st) {
+  if (d.o > 64) return false;
+  const int BB = unpack_chunk(d);
+  int op = d.o * d.o + 1;
+  if ((size_t)2 * BB * op * sizeof(double) > 65536) op = d.o * d.o;
+  const size_t lds = sizeof(double) * (size_t)2 * BB * op;
+  const int chunks = (d.v - 1 + BB - 1) / BB;
+  hipLaunchKernelGGL((unpack_tiled_kernel<double, true>), dim3(d.v, std::max(chunks, 1), nvec), dim3(PT), lds, st, G1,
+                     W, ldw, W, ldw, d, nullptr, lay, BB, op, G2);
+  HIP_CHECK(hipGetLastError());
+  return true;
 }
 
 #define INST(T)                                                                                           \
