@@ -155,7 +155,7 @@ struct OccSet {
 };
 
 template <int OM, int VG, bool UP, bool DOWN>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, OM == 16 && VG == 1 ? 3 : 2)
 csf_occ_kernel(CsfGeo g, int nt, int sl, const double* __restrict__ X, const double* __restrict__ Oc,
                const double* __restrict__ eps, double* __restrict__ W, double* __restrict__ part,
                double* __restrict__ T2) {
@@ -519,13 +519,21 @@ void launch_csf_build_o(const double* O, const DimsK& d, double* out, hipStream_
   HIP_CHECK(hipGetLastError());
 }
 
+// vectors a wave of the occupied kernel takes together
+static int csf_occ_vectors(int o, int nv) { return o <= 16 && nv > 1 ? 2 : 1; }
+
 CsfPlan csf_plan(const DimsK& d, int nv) {
   CsfPlan p;
   const int o = d.o, v = d.v;
   const int rows = nv * o, waves = (rows + 15) / 16;
   // down: rows in groups of dw waves (4, or fewer when there are no more),
   // columns in equal splits of at most 13 blocks of 16, K split so that about
-  // two workgroups per CU are in flight
+  // two workgroups per CU are in flight, each with three slabs or more.  The
+  // split orders the sums.  From 2 to 24 slabs its time at small sizes is the
+  // same to 1 us, so three was taken, in even numbers of workgroups, as the
+  // order under which solver runs that amplify the last bit (iterations to
+  // 1e-7 of the uncoupled-guess block Davidson; partially re-orthogonalised
+  // Lanczos past the loss of orthogonality) stay closest to the NumPy oracle
   const int nb = (v + 15) / 16;
   p.dns = (nb + 12) / 13;
   p.dnb = (nb + p.dns - 1) / p.dns;
@@ -535,8 +543,14 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   p.dg = (waves + p.dw - 1) / p.dw;
   const CsfGeo g8 = csf_geo<double>(d, nv, 0, 0), g4 = csf_geo<float>(d, nv, 0, 0);
   const int64_t tiles = std::min((int64_t)(2 * g8.nch + g8.nchd), (int64_t)(2 * g4.nch + g4.nchd)) * o;
-  p.ds = (int)std::max<int64_t>(1, std::min<int64_t>(tiles / 3, 512 / ((int64_t)p.dg * p.dns)));
-  p.down_bytes = (size_t)p.ds * rows * v * sizeof(double);
+  p.ds = (int)std::max<int64_t>(1, std::min<int64_t>(tiles / 6 * 2, 512 / ((int64_t)p.dg * p.dns)));
+  // one pass for both directions where the rows fit two 16-row blocks and a
+  // slab's columns the registers, and every workgroup has work for two rounds
+  // (o=16, v=200: one vector 0.29 ms against 0.26 + 0.27 in two passes, two
+  // vectors 0.49 against 0.33 + 0.30; o=5, v=36, 83 chunks: 17 us against 15)
+  const int items = 2 * g4.nch + g4.nchd;
+  p.thin = (o <= 16 && rows <= 32 && v <= 208 && items >= 512) ? 256 : 0;
+  p.down_bytes = (size_t)std::max(p.ds, p.thin) * rows * v * sizeof(double);
   // up: whole vectors per workgroup, the number of waves that pads least
   const int wmax = o <= 16 ? 8 : 4;
   double best = 1e300;
@@ -553,15 +567,17 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   }
   p.nt = nb;
   // occupied: slices of the sets so that the workgroups come in whole rounds
-  // of two per CU (their registers allow two); the fewest slices among equals
-  const int vgl = o <= 16 ? 2 : 1, vgs = (nv + vgl - 1) / vgl;
+  // of two per CU (three with one vector each: their registers); the fewest
+  // slices among equals
+  const int vgl = csf_occ_vectors(o, nv), vgs = (nv + vgl - 1) / vgl;
+  const int64_t slots = o <= 16 && vgl == 1 ? 768 : 512;
   const int64_t wgs = (int64_t)(nb * (nb + 1) / 2 + 3) / 4 * vgs;
   double beff = 0.0;
   p.sl = 1;
-  for (int sl = 1; sl <= 16 && sl <= (int)(2 * d.npo + o + 3) / 4; ++sl) {
+  for (int sl = 1; sl <= 32 && sl <= (int)(2 * d.npo + o + 3) / 4; ++sl) {
     const int64_t n = wgs * sl;
     if (n > 2048 && sl > 1) break;
-    const double eff = (double)n / (double)((n + 511) / 512 * 512);
+    const double eff = (double)n / (double)((n + slots - 1) / slots * slots);
     if (eff > 1.03 * beff) {
       beff = eff;
       p.sl = sl;
@@ -585,26 +601,28 @@ CsfBytes csf_workspace(const DimsK& d, int nv) {
 
 void launch_csf_occ(const CsfGeo& g, const CsfPlan& p, const double* X, const double* Oc, const double* eps,
                     double* W, double* part, double* T2, bool up, bool down, hipStream_t st) {
-  if (g.o <= 16)
+  if (g.o <= 16 && csf_occ_vectors(g.o, g.nv) == 1)
+    occ_launch<16, 1>(g, p, X, Oc, eps, W, part, T2, up, down, st);
+  else if (g.o <= 16)
     occ_launch<16, 2>(g, p, X, Oc, eps, W, part, T2, up, down, st);
   else
     occ_launch<32, 1>(g, p, X, Oc, eps, W, part, T2, up, down, st);
 }
 
 template <class Acc>
-void launch_csf_reduce(const CsfGeo& g, const CsfPlan& p, const Acc* down, const double* occ, double* W,
+void launch_csf_reduce(const CsfGeo& g, const CsfPlan& p, int ndown, const Acc* down, const double* occ, double* W,
                        hipStream_t st) {
   const int64_t total = (int64_t)g.o * g.v * g.nv;
-  hipLaunchKernelGGL((csf_reduce_kernel<Acc>), dim3((unsigned)((total + 31) / 32)), dim3(256), 0, st, g, p.ds, down,
+  hipLaunchKernelGGL((csf_reduce_kernel<Acc>), dim3((unsigned)((total + 31) / 32)), dim3(256), 0, st, g, ndown, down,
                      p.sl * p.nt, occ, W);
   HIP_CHECK(hipGetLastError());
 }
 
 template void launch_csf_build_v<double>(const double*, const DimsK&, double*, hipStream_t);
 template void launch_csf_build_v<float>(const double*, const DimsK&, float*, hipStream_t);
-template void launch_csf_reduce<double>(const CsfGeo&, const CsfPlan&, const double*, const double*, double*,
+template void launch_csf_reduce<double>(const CsfGeo&, const CsfPlan&, int, const double*, const double*, double*,
                                         hipStream_t);
-template void launch_csf_reduce<float>(const CsfGeo&, const CsfPlan&, const float*, const double*, double*,
+template void launch_csf_reduce<float>(const CsfGeo&, const CsfPlan&, int, const float*, const double*, double*,
                                        hipStream_t);
 
 }  // namespace adc2g

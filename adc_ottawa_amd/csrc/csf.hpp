@@ -67,6 +67,7 @@ struct CsfPlan {
   int dw, dg, dns, dnb, ds;  // down: waves, row groups, column splits, 16-column blocks, K splits
   int uw, uvpb, ug;          // up: waves, vectors per workgroup, groups
   int nt, sl;                // occupied: 16-virtual tiles, set slices
+  int thin;                  // workgroups of the pass that does both directions, 0: separate passes
   size_t down_bytes, occ_bytes, t2_bytes;
 };
 CsfPlan csf_plan(const DimsK& d, int nv);
@@ -87,12 +88,16 @@ void launch_csf_down(const CsfGeo& g, const CsfPlan& p, const double* X, const d
                      const T* V, typename Mma<T>::Acc* part, hipStream_t st);
 // W1 += both partials.
 template <class Acc>
-void launch_csf_reduce(const CsfGeo& g, const CsfPlan& p, const Acc* down, const double* occ, double* W,
+void launch_csf_reduce(const CsfGeo& g, const CsfPlan& p, int ndown, const Acc* down, const double* occ, double* W,
                        hipStream_t st);
 // W2 += virtual up term.
 template <class T>
 void launch_csf_up(const CsfGeo& g, const CsfPlan& p, const double* X, const double* zeros, const T* V, double* W,
                    hipStream_t st);
+// Both virtual terms (thin plans): W2 += the up term, partials of the down term.
+template <class T>
+void launch_csf_thin(const CsfGeo& g, const CsfPlan& p, const double* X, const double* T2, const double* zeros,
+                     const T* V, double* W, typename Mma<T>::Acc* part, hipStream_t st);
 inline size_t csf_zeros(const DimsK& d) {
   return (size_t)std::max<int64_t>(d.npv + d.v, d.n1 + 16 * d.o) + 64;
 }

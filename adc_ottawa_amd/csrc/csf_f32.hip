@@ -8,4 +8,7 @@ template void launch_csf_down<float>(const CsfGeo&, const CsfPlan&, const double
 template void launch_csf_up<float>(const CsfGeo&, const CsfPlan&, const double*, const double*, const float*, double*,
                                  hipStream_t);
 
+template void launch_csf_thin<float>(const CsfGeo&, const CsfPlan&, const double*, const double*, const double*,
+                                   const float*, double*, float*, hipStream_t);
+
 }  // namespace adc2g

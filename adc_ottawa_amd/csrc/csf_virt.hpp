@@ -472,6 +472,259 @@ up_kernel(CsfGeo g, int vpb, int ug, const double* __restrict__ X, const double*
   }
 }
 
+// ---- both directions in one pass over the operand, for at most 32 rows
+// (vec,k): a few vectors read the operand faster than they use it (1 GB for
+// o=16, v=200 in FP64, against 0.1 ms of MFMAs for one vector), and both
+// directions read the same one.  One workgroup a CU takes (chunk, type) after
+// (chunk, type); its waves take the l of one by turns, each streaming its slabs
+// through two LDS slots of its own (no barrier in the slab loop), with the
+// down sums of all columns and the H of its l in registers.  The down sums of
+// the four waves are added at the end, the H exchanged in LDS after each
+// (chunk, type) as in the up kernel.
+template <class T, int NB, int NS, int TM>
+__global__ void __launch_bounds__(256, 1)
+thin_kernel(CsfGeo g, const double* __restrict__ X, const double* __restrict__ T2, const double* __restrict__ zeros,
+            const T* __restrict__ V, double* __restrict__ W, typename Mma<T>::Acc* __restrict__ part) {
+  typedef Mma<T> MT;
+  typedef typename MT::v4 v4;
+  typedef typename MT::Acc Acc;
+  constexpr int KS = 32 / (int)sizeof(T), P = 4 * KS, PB = 8 / (int)sizeof(T);
+  constexpr int SB = (NB + NS - 1) / NS;  // blocks s*NB/NS .. of slab part s, at most SB
+  constexpr int NLW = 4;                  // l of a wave: wave, wave + 4, ...
+  constexpr int R = 16 * TM;
+  static_assert(NS % 2 == 0, "slab parts alternate between two slots");
+  typedef T th __attribute__((ext_vector_type(KS / 2)));
+  typedef T tv __attribute__((ext_vector_type(PB)));
+  __shared__ __attribute__((aligned(1024))) char r0[4][SB * 2048];
+  __shared__ __attribute__((aligned(1024))) char r1[4][SB * 2048];
+  __shared__ T x1s[NB * 16 * R];
+  __shared__ Acc hx[16 * 16 * P];
+  __shared__ unsigned char tk[120], tl[120];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, gq = lane >> 4;
+  const int o = g.o, v = g.v, rows = g.nv * o;
+  const int nb = (v + 15) / 16;
+  const int items = 2 * g.nch + g.nchd;
+  const int wg = xcd_tile(blockIdx.x, gridDim.x);
+  const int it0 = uniform((int)((int64_t)items * wg / gridDim.x)), it1 = uniform((int)((int64_t)items * (wg + 1) / gridDim.x));
+  const int64_t slab = (int64_t)v * 128;
+  const int lane16 = lane * 16;
+
+  for (int kk = threadIdx.x; kk < o; kk += 256) {
+    int q = (int)po_index(kk, kk + 1, o);
+    for (int ll = kk + 1; ll < o; ++ll, ++q) {
+      tk[q] = (unsigned char)kk;
+      tl[q] = (unsigned char)ll;
+    }
+  }
+  for (int t = threadIdx.x; t < NB * 16 * R; t += 256) {
+    const int c = t / R, rr = t - c * R;
+    const int vv = rr / o, kk = rr - vv * o;
+    x1s[t] = (rr < rows && c < v) ? (T)X[g.ldx * vv + (int64_t)c * o + kk] : (T)0;
+  }
+  int vec[TM], kr[TM];
+  bool live[TM];
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int row = m * 16 + li;
+    live[m] = row < rows;
+    vec[m] = live[m] ? row / o : 0;
+    kr[m] = live[m] ? row - vec[m] * o : 0;
+  }
+  __syncthreads();
+  const int nl = wave < o ? (o - wave + 3) / 4 : 0;
+
+  // (chunk, type) `it`: is it diagonal, t5, and its first slab
+  auto decode = [&](int it, int& diag, int& t, int& ch) ADC2G_INLINE {
+    diag = it >= 2 * g.nch ? 1 : 0;
+    ch = diag ? it - 2 * g.nch : it >> 1;
+    t = diag ? 0 : it & 1;
+  };
+  auto dma = [&](int it, int il, int s, char* buf) ADC2G_INLINE {
+    int diag, t, ch;
+    decode(it, diag, t, ch);
+    const int64_t u = (diag ? (int64_t)2 * g.nch * o + (int64_t)ch * o : (int64_t)ch * 2 * o + t * o) + wave + 4 * il;
+    const Rsrc src = lds_source((const char*)V + u * slab);
+    const int b0 = s * NB / NS, b1 = min((s + 1) * NB / NS, nb);
+    for (int i = 2 * b0; i < 2 * b1; ++i) lds_copy(src, i * 1024, buf + (i - 2 * b0) * 1024, lane16);
+  };
+  double xr[TM][KS];
+  int left = 0, five = 0, lx = 0;
+  auto load_x = [&](int it, int il) ADC2G_INLINE {
+    int diag, t, ch;
+    decode(it, diag, t, ch);
+    const int l = wave + 4 * il;
+    left = (diag ? v : (int)g.npv) - ch * P;
+    five = t;
+    lx = l;
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      const int k = kr[m];
+      const double* e = zeros;
+      if (live[m]) {
+        if (l == k) {
+          const double* t2v = T2 + (int64_t)(vec[m] * o + k) * (g.npv + v);
+          e = diag ? t2v + g.npv : (t ? zeros : t2v);
+        } else {
+          const int64_t q = po_index(min(k, l), max(k, l), o);
+          e = X + g.ldx * vec[m] + (diag ? g.off3 + q * v : (t ? g.off5 : g.off4) + q * g.npv);
+        }
+      }
+      e += ch * P;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int p = gq * KS + s;
+        xr[m][s] = e[p < left ? p : 0];
+      }
+    }
+  };
+  v4 sacc[TM][NB];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) sacc[m][j] = (v4){0, 0, 0, 0};
+  v4 h[NLW][TM][PB];
+  const int pa = li * 128 + (((2 * gq) ^ (li & 7)) << 4), pb = li * 128 + (((2 * gq + 1) ^ (li & 7)) << 4);
+  const int pu = (((li >> 1) << 4) | ((li & 1) << 3));
+
+  const int npo = g.npo;
+  if (nl > 0 && it0 < it1) {
+    load_x(it0, 0);
+    dma(it0, 0, 0, r0[wave]);
+  }
+  for (int it = it0; it < it1; ++it) {
+    int diag, t, ch;
+    decode(it, diag, t, ch);
+#pragma unroll
+    for (int il = 0; il < NLW; ++il) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int j = 0; j < PB; ++j) h[il][m][j] = (v4){0, 0, 0, 0};
+      if (il < nl) {
+        T a[TM][KS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this part (and the rows) have landed
+          __builtin_amdgcn_wave_barrier();
+          if (s == 0) {
+#pragma unroll
+            for (int m = 0; m < TM; ++m) {
+              const double sg = five && lx < kr[m] ? -1.0 : 1.0;
+#pragma unroll
+              for (int e = 0; e < KS; ++e) a[m][e] = gq * KS + e < left ? (T)(sg * xr[m][e]) : (T)0;
+            }
+          }
+          char* nxt = (s & 1) ? r0[wave] : r1[wave];
+          if (s + 1 < NS) {
+            dma(it, il, s + 1, nxt);
+          } else {
+            const int il2 = il + 1 < nl ? il + 1 : 0, it2 = il + 1 < nl ? it : it + 1;
+            if (it2 < it1) {
+              load_x(it2, il2);
+              dma(it2, il2, 0, nxt);
+            }
+          }
+          const char* cur = (s & 1) ? r1[wave] : r0[wave];
+#pragma unroll
+          for (int jj = 0; jj < SB; ++jj) {
+            const int j = s * NB / NS + jj;
+            if (j < (s + 1) * NB / NS && j < nb) {
+              const char* blk = cur + jj * 2048;
+              const th lo = *(const th*)(blk + pa), hi = *(const th*)(blk + pb);
+#pragma unroll
+              for (int e = 0; e < KS; ++e)
+#pragma unroll
+                for (int m = 0; m < TM; ++m)
+                  sacc[m][j] = MT::mma(a[m][e], e < KS / 2 ? lo[e % (KS / 2)] : hi[e % (KS / 2)], sacc[m][j]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int c = 4 * e + gq;
+                const tv b = *(const tv*)(blk + c * 128 + (pu ^ ((c & 7) << 4)));
+#pragma unroll
+                for (int m = 0; m < TM; ++m) {
+                  const T x = x1s[(j * 16 + c) * R + m * 16 + li];
+#pragma unroll
+                  for (int q = 0; q < PB; ++q) h[il][m][q] = MT::mma(x, b[q], h[il][m][q]);
+                }
+              }
+            }
+          }
+        }
+      }
+    }
+    // exchange, one vector at a time: hx[k][l][p]
+    const int p0 = ch * P;
+    const int np = min(P, (diag ? v : (int)g.npv) - p0);
+    for (int vv = 0; vv < g.nv; ++vv) {
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int rr = m * 16 + MT::row(lane, r);
+          const int kk = rr - vv * o;
+          if (kk < 0 || kk >= o) continue;
+#pragma unroll
+          for (int il = 0; il < NLW; ++il)
+            if (il < nl)
+#pragma unroll
+              for (int q = 0; q < PB; ++q) hx[(kk * o + wave + 4 * il) * P + PB * li + q] = h[il][m][q][r];
+        }
+      __syncthreads();
+      double* wv = W + g.ldw * vv;
+      const int p = threadIdx.x & (P - 1), y = threadIdx.x / P;
+      constexpr int NY = 256 / P;
+      if (p < np) {
+        double* wq = wv + (diag ? g.off3 : (t ? g.off5 : g.off4)) + p0 + p;
+        const int64_t sq = diag ? (int64_t)v : g.npv;
+        for (int q0 = y; q0 < npo; q0 += 8 * NY) {
+          double old[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) old[e] = wq[min(q0 + e * NY, npo - 1) * sq];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int q = q0 + e * NY;
+            if (q >= npo) break;
+            const int kk = tk[q], ll = tl[q];
+            const double h1 = (double)hx[(kk * o + ll) * P + p], h2 = (double)hx[(ll * o + kk) * P + p];
+            wq[q * sq] = old[e] + (t ? h1 - h2 : h1 + h2);
+          }
+        }
+      }
+      if (!t)
+        for (int i = threadIdx.x; i < np * o; i += 256) {
+          const int kk = diag ? i / np : i % o, pp = diag ? i % np : i / o;
+          double* w2 = diag ? wv + g.off1 + (int64_t)kk * v + p0 + pp : wv + g.off2 + (int64_t)p0 * o + i;
+          *w2 -= SQ2 * (double)hx[(kk * o + kk) * P + pp];
+        }
+    }
+  }
+  // down sums of the four waves, 16 rows at a time through the first slot
+  static_assert(NB * 16 * 16 * (int)sizeof(Acc) <= (int)sizeof(hx), "the sums fit the exchange buffer");
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    for (int w = 0; w < 4; ++w) {
+      __syncthreads();
+      if (wave == w) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            Acc* e = hx + MT::row(lane, r) * (NB * 16) + j * 16 + li;
+            *e = (w == 0 ? (Acc)0 : *e) + sacc[m][j][r];
+          }
+      }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 16 * v; i += 256) {
+      const int rr = i / v, c = i - rr * v;
+      if (m * 16 + rr < rows) part[((int64_t)wg * rows + m * 16 + rr) * v + c] = hx[rr * (NB * 16) + c];
+    }
+  }
+}
+
 template <class T, int NB>
 void down_launch(const CsfGeo& g, const CsfPlan& p, const double* X, const double* T2, const double* zeros, const T* V,
                  typename Mma<T>::Acc* part, hipStream_t st) {
@@ -500,6 +753,20 @@ void up_launch(const CsfGeo& g, const CsfPlan& p, const double* X, const double*
   HIP_CHECK(hipGetLastError());
 }
 
+template <class T, int TM>
+void thin_launch(const CsfGeo& g, const CsfPlan& p, const double* X, const double* T2, const double* zeros, const T* V,
+                 double* W, typename Mma<T>::Acc* part, hipStream_t st) {
+  const dim3 grid((unsigned)p.thin), blk(256);
+  const int nb = (g.v + 15) / 16;
+  if (nb <= 4)
+    hipLaunchKernelGGL((thin_kernel<T, 4, 2, TM>), grid, blk, 0, st, g, X, T2, zeros, V, W, part);
+  else if (nb <= 8)
+    hipLaunchKernelGGL((thin_kernel<T, 8, 2, TM>), grid, blk, 0, st, g, X, T2, zeros, V, W, part);
+  else
+    hipLaunchKernelGGL((thin_kernel<T, 13, 4, TM>), grid, blk, 0, st, g, X, T2, zeros, V, W, part);
+  HIP_CHECK(hipGetLastError());
+}
+
 }  // namespace csfv
 
 template <class T>
@@ -512,6 +779,15 @@ template <class T>
 void launch_csf_up(const CsfGeo& g, const CsfPlan& p, const double* X, const double* zeros, const T* V, double* W,
                    hipStream_t st) {
   csfv::up_launch<T, CSF_OMAX>(g, p, X, zeros, V, W, st);
+}
+
+template <class T>
+void launch_csf_thin(const CsfGeo& g, const CsfPlan& p, const double* X, const double* T2, const double* zeros,
+                     const T* V, double* W, typename Mma<T>::Acc* part, hipStream_t st) {
+  if (g.nv * g.o <= 16)
+    csfv::thin_launch<T, 1>(g, p, X, T2, zeros, V, W, part, st);
+  else
+    csfv::thin_launch<T, 2>(g, p, X, T2, zeros, V, W, part, st);
 }
 
 }  // namespace adc2g

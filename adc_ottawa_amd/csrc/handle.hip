@@ -728,11 +728,18 @@ void Handle::sigma_csf(const double* Xc, int64_t ldx, double* Wc, int64_t ldw, i
   hipEvent_t e = span(2, (double)nc * d.n2 * 8.0 * (up ? 2.0 : 1.0));
   launch_csf_occ(g, p, Xc, cs_O.get(), eps.get(), Wc, (double*)ws_pocc, (double*)ws_pt2, up, down, s);
   end(e);
+  if (p.thin && down && up) {
+    e = span(0, 2.0 * flops_v);
+    launch_csf_thin<T>(g, p, Xc, (const double*)ws_pt2, cs_zeros.get(), V, Wc, (Acc*)ws_pdown, s);
+    end(e);
+    launch_csf_reduce<Acc>(g, p, p.thin, (const Acc*)ws_pdown, (const double*)ws_pocc, Wc, s);
+    return;
+  }
   if (down) {
     e = span(0, flops_v);
     launch_csf_down<T>(g, p, Xc, (const double*)ws_pt2, cs_zeros.get(), V, (Acc*)ws_pdown, s);
     end(e);
-    launch_csf_reduce<Acc>(g, p, (const Acc*)ws_pdown, (const double*)ws_pocc, Wc, s);
+    launch_csf_reduce<Acc>(g, p, p.ds, (const Acc*)ws_pdown, (const double*)ws_pocc, Wc, s);
   }
   if (up) {
     e = span(0, flops_v);
