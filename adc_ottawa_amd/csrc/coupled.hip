@@ -169,70 +169,146 @@ __global__ void __launch_bounds__(CP_THREADS) cp_unit_pairs_kernel(int o, int v,
   }
 }
 
-// The same tensor with one workgroup per (c, vec): every V value its o rows
-// read -- R[x] = V[c][a'][x] for x = (b,l) and S[b][m] = V[b][a'][c o + m] --
-// is staged in LDS by coalesced loads (the per-row kernel above gathers the
+// The same tensor with one workgroup per c and CP_VECS vectors: every V value
+// their rows read -- R[x] = V[c][a'][x] for x = (b,l) and S[b][m] =
+// V[b][a'][c o + m] -- is staged in LDS once per a' by coalesced loads (the per-row kernel above gathers the
 // l = k' and b-strided terms one element per cache line), then the o rows
-// of n1 elements are written in order.  Each thread walks its (b, l) by a
-// fixed stride (no integer division per element), and the BF16/FP32 tensors
-// are formed in FP32 arithmetic (their rounding is coarser than its error).
-// LDS: (2 n1 + nbas) doubles.
-template <class T>
-__global__ void __launch_bounds__(CP_THREADS) cp_unit_pairs_lds_kernel(int o, int v, int nb, int j0,
+// of n1 elements are written in order.  The BF16/FP32 tensors are formed in
+// FP32 arithmetic (their rounding is coarser than its error).
+// LDS: (2 v os + o^2 + nbas) doubles, rows of os (odd, so that the reads down a
+// column of fixed l spread over the banks; os = o where that does not fit).
+//
+// A row with k != k' and c != a' is zero but for l = k' and b = a': a thread
+// takes W consecutive elements (one 16-byte store; W = 1 where a row is not a
+// multiple of that), computes at most the one with l = k', and the o x o
+// elements with b = a' follow in a second pass (in the first, one wave in six
+// of each row would run all its elements for them).  The writes bound it then: o = 16, v = 200, 64 vectors in BF16
+// (1.3 GB) @@TIME@@ one element at a time with every condition.
+constexpr int CP_VECS = 4;  // 3200 workgroups at o = 16, v = 200, 64 vectors
+constexpr int UP_THREADS = 512;  // two workgroups per CU by their LDS: four waves per SIMD
+
+template <class T, int W>
+__global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, int v, int os, int nb, int j0,
                                                                        const double* __restrict__ V,
                                                                        const double* __restrict__ O,
                                                                        const double* __restrict__ eps, double sigma,
                                                                        T* __restrict__ Z) {
   typedef typename std::conditional<std::is_same<T, double>::value, double, float>::type C;
+  typedef T Tw __attribute__((ext_vector_type(W)));
   extern __shared__ double sm[];
   const int n1 = o * v;
   double* R = sm;
-  double* S = sm + n1;
-  double* ev = S + n1;
-  const int vec = blockIdx.x % nb, c = blockIdx.x / nb;
-  const int j = j0 + vec, ap = j / o, kp = j % o;
-  const double* vr = V + ((int64_t)c * v + ap) * n1;
-  for (int x = threadIdx.x; x < n1; x += CP_THREADS) R[x] = vr[x];
-  for (int t = threadIdx.x; t < n1; t += CP_THREADS) {
-    const int b = t / o, m = t - b * o;
-    S[t] = V[((int64_t)b * v + ap) * n1 + (int64_t)c * o + m];
-  }
-  for (int t = threadIdx.x; t < o + v; t += CP_THREADS) ev[t] = eps[t];
-  __syncthreads();
-  const int qs = CP_THREADS / o, rs = CP_THREADS - qs * o;  // the stride CP_THREADS as (b, l) steps
-  const int b0 = threadIdx.x / o, l0 = threadIdx.x - b0 * o;
-  for (int k = 0; k < o; ++k) {
-    T* zr = Z + ((int64_t)(c * nb + vec) * o + k) * n1;
-    const C base = (C)(ev[o + c] - ev[k] - sigma);
-    int b = b0, l = l0;
-    for (int bl = threadIdx.x; bl < n1; bl += CP_THREADS) {
+  double* S = sm + v * os;
+  double* Q = S + v * os;  // Q[k][l] = O[k][k'][c o + l] = (k k'|c l)
+  double* ev = Q + o * o;
+  const int ng = (nb + CP_VECS - 1) / CP_VECS;
+  const int c = blockIdx.x / ng, vec0 = (blockIdx.x - c * ng) * CP_VECS, vec1 = min(nb, vec0 + CP_VECS);
+  for (int t = threadIdx.x; t < o + v; t += UP_THREADS) ev[t] = eps[t];
+  const int step = UP_THREADS * W, qs = step / o, rs = step - qs * o;  // a step as (b, l)
+  const int b0 = threadIdx.x * W / o, l0 = threadIdx.x * W - b0 * o;
+  int staged = -1;
+  for (int vec = vec0; vec < vec1; ++vec) {
+    const int j = j0 + vec, ap = j / o, kp = j - ap * o;
+    __syncthreads();
+    if (ap != staged) {
+      const double* vr = V + ((int64_t)c * v + ap) * n1;
+      for (int t = threadIdx.x; t < n1; t += UP_THREADS) {
+        const int b = t / o, m = t - b * o;
+        R[b * os + m] = vr[t];
+        S[b * os + m] = V[((int64_t)b * v + ap) * n1 + (int64_t)c * o + m];
+      }
+      staged = ap;
+    }
+    for (int t = threadIdx.x; t < o * o; t += UP_THREADS) {
+      const int k = t / o;
+      Q[t] = O[((int64_t)k * o + kp) * n1 + (int64_t)c * o + (t - k * o)];
+    }
+    __syncthreads();
+    T* zv = Z + (int64_t)(c * nb + vec) * o * n1;
+    auto element = [&](int k, int b, int l) -> T {
       double g1 = 0.0, g2 = 0.0, g3 = 0.0, g4 = 0.0;
       if (k == kp) {
-        g1 += R[bl];          // (c a'|b l)
-        g3 += S[b * o + l];   // (b a'|c l)
+        g1 += R[b * os + l];  // (c a'|b l)
+        g3 += S[b * os + l];  // (b a'|c l)
       }
       if (c == ap) {
-        g1 -= O[((int64_t)k * o + kp) * n1 + bl];                  // (k k'|b l)
+        g1 -= O[((int64_t)k * o + kp) * n1 + (int64_t)b * o + l];  // (k k'|b l)
         g4 -= O[((int64_t)l * o + kp) * n1 + (int64_t)b * o + k];  // (l k'|b k)
       }
       if (l == kp) {
-        g2 += S[b * o + k];   // (b a'|c k)
-        g4 += R[b * o + k];   // (c a'|b k)
+        g2 += S[b * os + k];  // (b a'|c k)
+        g4 += R[b * os + k];  // (c a'|b k)
       }
       if (b == ap) {
-        g2 -= O[((int64_t)l * o + kp) * n1 + (int64_t)c * o + k];  // (l k'|c k)
-        g3 -= O[((int64_t)k * o + kp) * n1 + (int64_t)c * o + l];  // (k k'|c l)
+        g2 -= Q[l * o + k];  // (l k'|c k)
+        g3 -= Q[k * o + l];  // (k k'|c l)
       }
       const C num = (C)(2.0 * g1 + 2.0 * g2 - g3 - g4);
-      zr[bl] = (T)(num / (base + (C)(ev[o + b] - ev[l])));
+      return (T)(num / ((C)(ev[o + c] - ev[k] - sigma) + (C)(ev[o + b] - ev[l])));
+    };
+    int k = 0, b = b0, l = l0;
+    while (b >= v) {
+      b -= v;
+      ++k;
+    }
+    for (int bl = threadIdx.x * W; bl < o * n1; bl += step) {
+      Tw z;
+      if (k == kp || c == ap || o < W) {
+        int be = b, le = l;
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+          z[e] = element(k, be, le);
+          if (++le == o) {
+            le = 0;
+            ++be;
+          }
+        }
+      } else {
+        // the elements of the l range [l, l + W) mod o, o >= W: k' once at most
+        const bool wrap = kp < l;
+        const int es = wrap ? kp + o - l : kp - l;
+        T x = (T)0;
+        if (es < W) {
+          const int be = wrap ? b + 1 : b;
+          const C num = (C)(2.0 * S[be * os + k] - R[be * os + k]);
+          x = (T)(num / ((C)(ev[o + c] - ev[k] - sigma) + (C)(ev[o + be] - ev[kp])));
+        }
+#pragma unroll
+        for (int e = 0; e < W; ++e) z[e] = e == es ? x : (T)0;
+      }
+      *(Tw*)(zv + bl) = z;
       l += rs;
       b += qs;
       if (l >= o) {
         l -= o;
         ++b;
       }
+      while (b >= v) {
+        b -= v;
+        ++k;
+      }
+    }
+    if (c != ap && o >= W) {
+      __syncthreads();  // over the zeros of other threads
+      for (int t = threadIdx.x; t < o * o; t += UP_THREADS) {
+        const int kk = t / o, ll = t - kk * o;
+        if (kk != kp) zv[(int64_t)kk * n1 + ap * o + ll] = element(kk, ap, ll);
+      }
     }
   }
+}
+
+template <class T>
+void unit_pairs_lds(int o, int v, int nb, int j0, const double* V, const double* O, const double* eps, double sigma,
+                    T* Z, hipStream_t st) {
+  constexpr int W = 16 / (int)sizeof(T);
+  auto bytes = [&](int os) { return sizeof(double) * ((size_t)2 * v * os + o * o + o + v); };
+  const int os = bytes(o | 1) <= 65536 ? (o | 1) : o;
+  const dim3 grid((unsigned)v * ((nb + CP_VECS - 1) / CP_VECS)), blk(UP_THREADS);
+  if ((o * v) % W == 0)
+    hipLaunchKernelGGL((cp_unit_pairs_lds_kernel<T, W>), grid, blk, bytes(os), st, o, v, os, nb, j0, V, O, eps, sigma, Z);
+  else
+    hipLaunchKernelGGL((cp_unit_pairs_lds_kernel<T, 1>), grid, blk, bytes(os), st, o, v, os, nb, j0, V, O, eps, sigma, Z);
 }
 
 // A[:, j0 + c] = H11[:, j0 + c] - M[:, c] (n1 x nb; H11 symmetric)
@@ -329,23 +405,14 @@ void CoupledPrecon::form_schur(double s, Prec bp) {
     const int o = Hd.d.o, v = Hd.d.v;
     for (int j0 = 0; j0 < n1; j0 += nc) {
       const int nb = std::min(nc, n1 - j0);
-      // staged variant when its LDS fits 64 KB (o = 16, v = 200: 52 KB)
-      const size_t lds = sizeof(double) * ((size_t)2 * n1 + o + v);
+      // staged variant when its LDS fits 64 KB (o = 16, v = 200: 58 KB with
+      // padded rows)
+      const size_t lds = sizeof(double) * ((size_t)2 * n1 + o * o + o + v);
       if (lds <= 65536) {
-        const dim3 grid((unsigned)v * nb);
         switch (bp) {
-          case Prec::F64:
-            hipLaunchKernelGGL(cp_unit_pairs_lds_kernel<double>, grid, blk, lds, st, o, v, nb, j0, V, O, Hd.eps.get(),
-                               sigma, (double*)Hd.ZG.get());
-            break;
-          case Prec::F32:
-            hipLaunchKernelGGL(cp_unit_pairs_lds_kernel<float>, grid, blk, lds, st, o, v, nb, j0, V, O, Hd.eps.get(),
-                               sigma, (float*)Hd.ZG.get());
-            break;
-          case Prec::BF16:
-            hipLaunchKernelGGL(cp_unit_pairs_lds_kernel<__bf16>, grid, blk, lds, st, o, v, nb, j0, V, O,
-                               Hd.eps.get(), sigma, (__bf16*)Hd.ZG.get());
-            break;
+          case Prec::F64: unit_pairs_lds(o, v, nb, j0, V, O, Hd.eps.get(), sigma, (double*)Hd.ZG.get(), st); break;
+          case Prec::F32: unit_pairs_lds(o, v, nb, j0, V, O, Hd.eps.get(), sigma, (float*)Hd.ZG.get(), st); break;
+          case Prec::BF16: unit_pairs_lds(o, v, nb, j0, V, O, Hd.eps.get(), sigma, (__bf16*)Hd.ZG.get(), st); break;
         }
       } else {
         const dim3 grid((unsigned)v * nb * o);

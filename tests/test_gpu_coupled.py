@@ -41,6 +41,24 @@ def test_schur_vs_oracle(form, o, v, naux, seed):
     assert np.abs(a64 - a64.T).max() == 0.0
 
 
+# nocc below and above the elements of a 16-byte store (2 | 4 | 8), rows that are
+# and are not multiples of it, groups that wrap from one b to the next, the last
+# vector chunk partial; 240: the largest rows that are staged, unpadded
+@pytest.mark.parametrize("o,v", [(2, 8), (2, 9), (3, 8), (7, 16), (8, 10), (9, 9), (12, 14), (16, 33), (17, 24), (16, 240)])
+def test_schur_pair_tensor_edges(o, v):
+    print(f"[case] coupled schur pair tensors o={o} v={v}", flush=True)
+    sys_ = make_system(o, v, 12, seed=o + v)
+    sig = 2.0 * (sys_.eps[o:].min() - sys_.eps[:o].max()) - 0.3
+    with lib.Operator.from_system(sys_, coupling="df") as op:
+        ref = op.coupled_schur(sig, precision="fp64")
+    scale = np.abs(ref).max()
+    with lib.Operator.from_system(sys_, coupling="int") as op:
+        # BF16: both operands of a product are within 2^-9 of their values
+        for prec, tol in (("fp64", 1e-11), ("fp32", 1e-5), ("bf16", 2.0 ** -8)):
+            a = op.coupled_schur(sig, precision=prec)
+            assert np.abs(a - ref).max() < tol * scale
+
+
 @pytest.fixture(scope="module")
 def water():
     print("[case] coupled davidson water-size o=5 v=36 naux=164", flush=True)
