@@ -171,19 +171,22 @@ __global__ void __launch_bounds__(CP_THREADS) cp_unit_pairs_kernel(int o, int v,
 
 // The same tensor with one workgroup per c and CP_VECS vectors: every V value
 // their rows read -- R[x] = V[c][a'][x] for x = (b,l) and S[b][m] =
-// V[b][a'][c o + m] -- is staged in LDS once per a' by coalesced loads (the per-row kernel above gathers the
-// l = k' and b-strided terms one element per cache line), then the o rows
-// of n1 elements are written in order.  The BF16/FP32 tensors are formed in
-// FP32 arithmetic (their rounding is coarser than its error).
-// LDS: (2 v os + o^2 + nbas) doubles, rows of os (odd, so that the reads down a
-// column of fixed l spread over the banks; os = o where that does not fit).
+// V[b][a'][c o + m] -- is staged in LDS once per a' by coalesced loads (the
+// per-row kernel above gathers the l = k' and b-strided terms one element per
+// cache line), then the o rows of n1 elements are written in order.  The
+// BF16/FP32 tensors are formed in FP32 arithmetic (their rounding is coarser
+// than its error).  LDS: (2 v os + nbas) doubles, rows of os (odd, so that the
+// reads down a column of fixed l spread over the banks; os = o where that does
+// not fit).
 //
-// A row with k != k' and c != a' is zero but for l = k' and b = a': a thread
+// A row with k != k' and c != a' is zero but for l = k' and b = a'.  A thread
 // takes W consecutive elements (one 16-byte store; W = 1 where a row is not a
-// multiple of that), computes at most the one with l = k', and the o x o
-// elements with b = a' follow in a second pass (in the first, one wave in six
-// of each row would run all its elements for them).  The writes bound it then: o = 16, v = 200, 64 vectors in BF16
-// (1.3 GB) @@TIME@@ one element at a time with every condition.
+// multiple of that) and computes at most the one with l = k'; the o x o
+// elements with b = a' follow in a second pass, since in the first a wave that
+// meets one would run all its elements and wait for their integrals in turn.
+// Then the writes bound it: o = 16, v = 200, 64 vectors in BF16 (1.3 GB) take
+// 0.47 ms (2.8 TB/s); one element at a time with every condition and one vector
+// per workgroup took 1.14 ms.
 constexpr int CP_VECS = 4;  // 3200 workgroups at o = 16, v = 200, 64 vectors
 constexpr int UP_THREADS = 512;  // two workgroups per CU by their LDS: four waves per SIMD
 
@@ -199,8 +202,7 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
   const int n1 = o * v;
   double* R = sm;
   double* S = sm + v * os;
-  double* Q = S + v * os;  // Q[k][l] = O[k][k'][c o + l] = (k k'|c l)
-  double* ev = Q + o * o;
+  double* ev = S + v * os;
   const int ng = (nb + CP_VECS - 1) / CP_VECS;
   const int c = blockIdx.x / ng, vec0 = (blockIdx.x - c * ng) * CP_VECS, vec1 = min(nb, vec0 + CP_VECS);
   for (int t = threadIdx.x; t < o + v; t += UP_THREADS) ev[t] = eps[t];
@@ -219,13 +221,10 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
       }
       staged = ap;
     }
-    for (int t = threadIdx.x; t < o * o; t += UP_THREADS) {
-      const int k = t / o;
-      Q[t] = O[((int64_t)k * o + kp) * n1 + (int64_t)c * o + (t - k * o)];
-    }
     __syncthreads();
     T* zv = Z + (int64_t)(c * nb + vec) * o * n1;
-    auto element = [&](int k, int b, int l) -> T {
+    const bool two = c != ap && o >= W;  // b = a' in the second pass
+    auto element = [&](int k, int b, int l, bool at_ap) -> T {
       double g1 = 0.0, g2 = 0.0, g3 = 0.0, g4 = 0.0;
       if (k == kp) {
         g1 += R[b * os + l];  // (c a'|b l)
@@ -239,9 +238,9 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
         g2 += S[b * os + k];  // (b a'|c k)
         g4 += R[b * os + k];  // (c a'|b k)
       }
-      if (b == ap) {
-        g2 -= Q[l * o + k];  // (l k'|c k)
-        g3 -= Q[k * o + l];  // (k k'|c l)
+      if (at_ap) {
+        g2 -= O[((int64_t)l * o + kp) * n1 + (int64_t)c * o + k];  // (l k'|c k)
+        g3 -= O[((int64_t)k * o + kp) * n1 + (int64_t)c * o + l];  // (k k'|c l)
       }
       const C num = (C)(2.0 * g1 + 2.0 * g2 - g3 - g4);
       return (T)(num / ((C)(ev[o + c] - ev[k] - sigma) + (C)(ev[o + b] - ev[l])));
@@ -253,11 +252,11 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
     }
     for (int bl = threadIdx.x * W; bl < o * n1; bl += step) {
       Tw z;
-      if (k == kp || c == ap || o < W) {
+      if (k == kp || !two) {
         int be = b, le = l;
 #pragma unroll
         for (int e = 0; e < W; ++e) {
-          z[e] = element(k, be, le);
+          z[e] = element(k, be, le, !two && be == ap);
           if (++le == o) {
             le = 0;
             ++be;
@@ -288,11 +287,11 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
         ++k;
       }
     }
-    if (c != ap && o >= W) {
-      __syncthreads();  // over the zeros of other threads
+    if (two) {
+      __syncthreads();  // over the first pass
       for (int t = threadIdx.x; t < o * o; t += UP_THREADS) {
         const int kk = t / o, ll = t - kk * o;
-        if (kk != kp) zv[(int64_t)kk * n1 + ap * o + ll] = element(kk, ap, ll);
+        zv[(int64_t)kk * n1 + ap * o + ll] = element(kk, ap, ll, true);
       }
     }
   }
@@ -302,7 +301,7 @@ template <class T>
 void unit_pairs_lds(int o, int v, int nb, int j0, const double* V, const double* O, const double* eps, double sigma,
                     T* Z, hipStream_t st) {
   constexpr int W = 16 / (int)sizeof(T);
-  auto bytes = [&](int os) { return sizeof(double) * ((size_t)2 * v * os + o * o + o + v); };
+  auto bytes = [&](int os) { return sizeof(double) * ((size_t)2 * v * os + o + v); };
   const int os = bytes(o | 1) <= 65536 ? (o | 1) : o;
   const dim3 grid((unsigned)v * ((nb + CP_VECS - 1) / CP_VECS)), blk(UP_THREADS);
   if ((o * v) % W == 0)
@@ -405,9 +404,9 @@ void CoupledPrecon::form_schur(double s, Prec bp) {
     const int o = Hd.d.o, v = Hd.d.v;
     for (int j0 = 0; j0 < n1; j0 += nc) {
       const int nb = std::min(nc, n1 - j0);
-      // staged variant when its LDS fits 64 KB (o = 16, v = 200: 58 KB with
+      // staged variant when its LDS fits 64 KB (o = 16, v = 200: 56 KB with
       // padded rows)
-      const size_t lds = sizeof(double) * ((size_t)2 * n1 + o * o + o + v);
+      const size_t lds = sizeof(double) * ((size_t)2 * n1 + o + v);
       if (lds <= 65536) {
         switch (bp) {
           case Prec::F64: unit_pairs_lds(o, v, nb, j0, V, O, Hd.eps.get(), sigma, (double*)Hd.ZG.get(), st); break;
