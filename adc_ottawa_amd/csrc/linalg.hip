@@ -20,6 +20,42 @@ constexpr int SYEV_NMAX = 512;
 constexpr int SYEVX_ZCAP = 10240;  // doubles of LDS for the eigenvector block (80 KB)
 constexpr int ORTH_ZCAP = 4096;    // the same for the Gram-matrix eigensolve (blocks up to 64)
 
+// x plus the x of lane ^ OFF.  A full wave only.  The pairs come by permlane
+// swaps and DPP moves, a few cycles each, where __shfl_xor goes through the LDS
+// crossbar; the sums are those of the butterfly over __shfl_xor, bit for bit.
+template <int CTRL>
+__device__ __forceinline__ int dpp_xor(int x) {
+  if (CTRL == 4) {  // lanes 0-3, 8-11 of a row from four up, the others from four down
+    const int t = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0x5, false);
+    return __builtin_amdgcn_update_dpp(t, x, 0x114, 0xf, 0xa, false);
+  }
+  constexpr int C = CTRL == 8 ? 0x128 : CTRL == 2 ? 0x4e : 0xb1;  // row_ror:8, quad_perm
+  return __builtin_amdgcn_update_dpp(x, x, C, 0xf, 0xf, false);
+}
+
+template <int OFF>
+__device__ __forceinline__ double add_xor(double x) {
+  const uint32_t l = (uint32_t)__double2loint(x), h = (uint32_t)__double2hiint(x);
+  if constexpr (OFF >= 16) {
+    const auto a = OFF == 32 ? __builtin_amdgcn_permlane32_swap(l, l, false, false)
+                             : __builtin_amdgcn_permlane16_swap(l, l, false, false);
+    const auto b = OFF == 32 ? __builtin_amdgcn_permlane32_swap(h, h, false, false)
+                             : __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+  } else {
+    return x + __hiloint2double(dpp_xor<OFF>((int)h), dpp_xor<OFF>((int)l));
+  }
+}
+
+__device__ __forceinline__ double wave_sum(double x) {
+  x = add_xor<32>(x);
+  x = add_xor<16>(x);
+  x = add_xor<8>(x);
+  x = add_xor<4>(x);
+  x = add_xor<2>(x);
+  return add_xor<1>(x);
+}
+
 __device__ double block_sum(double x, double* sh) {
   for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -46,7 +82,7 @@ struct SyevShared {
 // form p = A22 v (partials in S.rc), wave 0 forms q = 2 (p - (v.p) v) (S.qv),
 // all waves apply A22 <- A22 - v q^T - q v^T.  Zw is unused (kept for the
 // callers' workspace layout).
-__device__ void tridiag_dev(int n, double* A, int lda, double* Zw, SyevShared& S) {
+__device__ __forceinline__ void tridiag_dev(int n, double* A, int lda, double* Zw, SyevShared& S) {
   (void)Zw;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
@@ -58,7 +94,7 @@ __device__ void tridiag_dev(int n, double* A, int lda, double* Zw, SyevShared& S
     if (wv == 0) {
       double part = 0.0;
       for (int i = k + 2 + lane; i < n; i += 64) part += col[i] * col[i];
-      for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
+      part = wave_sum(part);
       const double x0 = col[k + 1];
       if (part == 0.0) {
         for (int i = k + 1 + lane; i < n; i += 64) vv[i] = 0.0;
@@ -113,7 +149,7 @@ __device__ void tridiag_dev(int n, double* A, int lda, double* Zw, SyevShared& S
           qv[i] = s;  // p for now
           kv += s * vv[i];
         }
-        for (int off = 32; off > 0; off >>= 1) kv += __shfl_xor(kv, off, 64);
+        kv = wave_sum(kv);
         for (int i = k + 1 + lane; i < n; i += 64) qv[i] = 2.0 * (qv[i] - kv * vv[i]);
       }
     }
@@ -237,7 +273,7 @@ __device__ void syev_dev(int n, double* A, int lda, double* w, double* Z, int ld
         const double* v = A + (int64_t)k * lda;
         double t = 0.0;
         for (int i = k + 1 + lane; i < n; i += 64) t += v[i] * z[i];
-        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        t = wave_sum(t);
         t *= 2.0;
         if (t != 0.0)
           for (int i = k + 1 + lane; i < n; i += 64) z[i] -= t * v[i];
@@ -316,11 +352,14 @@ __device__ __forceinline__ double unit_rand(uint64_t a, uint64_t b) {
 //  * back-transformation of the k vectors with the stored reflectors.
 // work: 2n + 6nk doubles.
 // zl / zcap: LDS for the k eigenvectors ([i * k + j]) through inverse
-// iteration, Gram-Schmidt and back-transformation when k * n <= zcap (their
-// steps are serial chains, so the latency of each access is what counts);
-// otherwise they run on Z in global memory.
-__device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z, int ldz, double* work, int* info,
-                          SyevShared& S, BisectShared& B, double* zl = nullptr, int zcap = 0) {
+// iteration, Gram-Schmidt and back-transformation when k * n <= zcap;
+// otherwise they run on Z in global memory.  ALL: A and the factors of the
+// inverse iteration are in LDS too (A, work; work without its first 2n), and
+// zl holds the eigenvectors whatever their number.
+template <bool ALL>
+__device__ __forceinline__ void syevx_steps(int n, int k, double* A, int lda, double* w, double* Z, int ldz,
+                                            double* work, int* info, SyevShared& S, BisectShared& B, double* zl,
+                                            int zcap) {
   const int tid = threadIdx.x, nt = blockDim.x;
   const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
   tridiag_dev(n, A, lda, work, S);
@@ -382,15 +421,21 @@ __device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z
     }
     __syncthreads();
     int open = 0;
-    for (int jj = tid; jj < k; jj += nt) {
+    for (int jj = wv; jj < k; jj += nw) {
       double lo = B.lo[jj], hi = B.hi[jj];
-      for (int gg = 0; gg < G; ++gg) {
+      for (int gg = lane; gg < G; gg += 64) {
         const double x = B.xs[jj * G + gg];
         if (B.cs[jj * G + gg] <= jj) lo = fmax(lo, x);
         else hi = fmin(hi, x);
       }
-      B.lo[jj] = lo;
-      B.hi[jj] = hi;
+      for (int off = 32; off > 0; off >>= 1) {
+        lo = fmax(lo, __shfl_xor(lo, off, 64));
+        hi = fmin(hi, __shfl_xor(hi, off, 64));
+      }
+      if (lane == 0) {
+        B.lo[jj] = lo;
+        B.hi[jj] = hi;
+      }
       const double tol = DBL_EPSILON * (2.0 * fmax(fabs(lo), fabs(hi)) + tnorm);
       const double mid = 0.5 * (lo + hi);
       if (hi - lo > tol && mid > lo && mid < hi) open = 1;
@@ -411,12 +456,12 @@ __device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z
   __syncthreads();
   // ---- inverse iteration, one lane per eigenvalue; arrays [i * k + j]
   {
-    double* U1 = work + 2 * n;
+    double* U1 = ALL ? work : work + 2 * n;
     double* U2 = U1 + (int64_t)n * k;
     double* U3 = U2 + (int64_t)n * k;
     double* ML = U3 + (int64_t)n * k;
     double* PV = ML + (int64_t)n * k;
-    double* Y = (zl && (int64_t)n * k <= zcap) ? zl : PV + (int64_t)n * k;
+    double* Y = ALL || (int64_t)n * k <= zcap ? zl : PV + (int64_t)n * k;
     const double tiny = DBL_EPSILON * tnorm;
     for (int j = tid; j < k; j += nt) {
       const double mu = B.mu[j];
@@ -477,13 +522,13 @@ __device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z
         const double sc = (ymax > 0.0 && isfinite(ymax)) ? 1.0 / ymax : 0.0;
         for (int i = 0; i < n; ++i) Y[(int64_t)i * k + j] *= sc;
       }
-      if (Y != zl)
+      if (!ALL && Y != zl)
         for (int i = 0; i < n; ++i) Z[i + (int64_t)j * ldz] = Y[(int64_t)i * k + j];
     }
   }
   __syncthreads();
   // element (i, j) of the eigenvector block: LDS or Z
-  const bool in_lds = zl && (int64_t)n * k <= zcap;
+  const bool in_lds = ALL || (int64_t)n * k <= zcap;
   auto zat = [&](int i, int j) -> double& { return in_lds ? zl[(int64_t)i * k + j] : Z[i + (int64_t)j * ldz]; };
   // ---- two modified Gram-Schmidt sweeps (wave 0)
   if (wv == 0) {
@@ -492,13 +537,13 @@ __device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z
         for (int i = 0; i < j; ++i) {
           double t = 0.0;
           for (int r = lane; r < n; r += 64) t += zat(r, i) * zat(r, j);
-          for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+          t = wave_sum(t);
           for (int r = lane; r < n; r += 64) zat(r, j) -= t * zat(r, i);
         }
       }
       double t = 0.0;
       for (int r = lane; r < n; r += 64) t += zat(r, j) * zat(r, j);
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+      t = wave_sum(t);
       const double sc = (t > 0.0) ? 1.0 / sqrt(t) : 0.0;
       for (int r = lane; r < n; r += 64) zat(r, j) *= sc;
     }
@@ -510,7 +555,7 @@ __device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z
       const double* v = A + (int64_t)kk * lda;
       double t = 0.0;
       for (int i = kk + 1 + lane; i < n; i += 64) t += v[i] * zat(i, j);
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+      t = wave_sum(t);
       t *= 2.0;
       if (t != 0.0)
         for (int i = kk + 1 + lane; i < n; i += 64) zat(i, j) -= t * v[i];
@@ -524,6 +569,28 @@ __device__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z
     }
   if (tid == 0) info[0] = 0;
   __syncthreads();
+}
+
+// Every step is a chain of dependent accesses on one workgroup, so their
+// latency is the time: with n^2 + 6nk doubles within zcap all of them are in
+// LDS, else the eigenvectors alone where they fit.  n up to 40, k = 5, mean
+// over a Davidson run: 156 us from global memory, 125 in LDS, 75 with the wave
+// sums above and a bracket's counts shared by a wave; the coefficients from a
+// Gram matrix of 5 vectors 83, 67 and 34 us.
+__device__ __forceinline__ void syevx_dev(int n, int k, double* A, int lda, double* w, double* Z, int ldz,
+                                          double* work, int* info, SyevShared& S, BisectShared& B, double* zl,
+                                          int zcap) {
+  if ((int64_t)n * n + 6 * (int64_t)n * k <= zcap) {
+    double* Al = zl + n * k;
+    for (int t = threadIdx.x; t < n * n; t += blockDim.x) {
+      const int j = t / n;
+      Al[t] = A[t - j * n + (int64_t)j * lda];
+    }
+    __syncthreads();
+    syevx_steps<true>(n, k, Al, n, w, Z, ldz, Al + n * n, info, S, B, zl, zcap);
+  } else {
+    syevx_steps<false>(n, k, A, lda, w, Z, ldz, work, info, S, B, zl, zcap);
+  }
 }
 
 __global__ void __launch_bounds__(SYEV_THREADS) syevx_kernel(int n, int k, double* A, int lda, double* w, double* Z,

@@ -151,3 +151,20 @@ def test_guess_errors(water):
     with pytest.raises(lib.Adc2gError) as e:
         op.davidson(5, blocksize=5, maxvec=40, guess="subdiag", subdim=3)   # blocksize > subdim
     assert e.value.code == 10
+
+
+# the subspace grows through the largest small eigenproblem that is solved in
+# LDS (n^2 + 6 n k = 10240 doubles) and, with 1 and 33 roots, through Gram
+# matrices on both sides of theirs (7 r^2 = 4096)
+@pytest.mark.parametrize("nroots,maxvec", [(1, 110), (4, 100), (9, 90), (24, 96), (33, 99)])
+def test_small_eigenproblem_storage(nroots, maxvec):
+    print(f"[case] davidson o=4 v=9 roots={nroots} maxvec={maxvec}", flush=True)
+    sys_ = make_system(4, 9, 20, seed=2)
+    lam = np.linalg.eigvalsh(elements.build_blocks(sys_, apply_minc=False).dense())
+    with lib.Operator.from_system(sys_) as op:
+        ev, X, st = op.davidson(nroots, blocksize=nroots, maxvec=maxvec, tol=1e-8, maxiter=400)
+        W = op.sigma(X)
+    # eigenvalue errors are of second order in residuals of 1e-8, over gaps of 1e-4 and more
+    assert np.abs(ev - lam[:nroots]).max() < 1e-10
+    assert np.linalg.norm(W - X * ev, axis=0).max() < 1.1e-8
+    assert np.abs(X.T @ X - np.eye(nroots)).max() < 1e-9
