@@ -18,7 +18,8 @@
 // index, so the vectors are read and written in their own order: the pair
 // tensor form moved n1^2 elements three times per direction beside them.  20
 // vectors at o=16, v=200: FP64 5.70 -> 3.81 ms, FP32 3.91 -> 2.59 ms; 7 vectors
-// at o=13, v=117: 0.61 -> 0.39 ms; one at o=5, v=36: 67 -> 43 us.
+// at o=13, v=117: 0.61 -> 0.39 ms; two at o=16, v=200: 0.92 -> 0.58 ms; one at
+// o=5, v=36: 67 -> 38 us.
 #include "csf.hpp"
 
 #include <algorithm>

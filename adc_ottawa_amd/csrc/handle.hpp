@@ -84,7 +84,8 @@ struct Handle {
   // optional per-kernel device timing of sigma-vectors (benchmark): event
   // pairs around the main coupling GEMMs (class 0: the virtual-index
   // contractions, or the naux contractions of the DF form), the CSF->pair
-  // packing (1), the pair->CSF projection with the 2h2p diagonal (2) and the
+  // packing (1; none on CSF vectors), the pair->CSF projection with the 2h2p
+  // diagonal, or on CSF vectors the occupied term with it (2), and the
   // remaining coupling GEMMs (3), with the algorithmic flops (classes 0, 3)
   // or bytes (1, 2) each launch is credited with.
   struct ProfRec {

@@ -304,10 +304,11 @@ int32_t adc2g_sigma_device(adc2g_handle* h, int32_t nvec, const double* dX, doub
  * graph capture, tight serving loops).  Every workspace (pair tensors, packed
  * 1h1p blocks, GEMM split-K partials) lies in one static device array of
  * 256 MiB per GPU that the library holds until the process ends; the vectors
- * go through it in passes of as many columns as fit (at o=16, v=200: 2 FP64,
- * 4 FP32 or 9 BF16 vectors per pass).  ADC2G_ENOMEM when one vector's
- * workspace does not fit (n1^2 elements of the precision plus its partials,
- * e.g. FP64 beyond n1 of about 4000); ADC2G_EARG for a CVS view or a
+ * go through it in passes of as many columns as fit (at o=16, v=200: 24 FP64
+ * or FP32 or 9 BF16 vectors per pass).  ADC2G_ENOMEM when one vector's
+ * workspace does not fit (in BF16, in the DF form and beyond 32 occupied
+ * orbitals n1^2 elements of the precision plus its partials; otherwise the
+ * partials, some hundred n1, and one copy of o rows of pairs); ADC2G_EARG for a CVS view or a
  * precision whose operands are not resident yet (create the handle with
  * keep_lowprec = 1, or run one adc2g_sigma_device of that precision first).
  * Calls on one GPU share the array: calls that overlap on one GPU race. */
@@ -706,7 +707,9 @@ int32_t adc2g_last_error(char* buf, int32_t len);
  * source/utilities/timingmod.f90:37-55).  enable = 1 starts recording HIP
  * events around the main coupling contractions (class 0: the sums over the
  * virtual index, or over naux in the DF form), the CSF -> pair-tensor packing
- * (class 1), the pair -> CSF projection fused with the 2h2p diagonal (class 2)
+ * (class 1; no launches in the INT form on CSF vectors), the pair -> CSF
+ * projection fused with the 2h2p diagonal, or on CSF vectors the occupied
+ * term with that diagonal (class 2)
  * and the remaining coupling contractions (class 3) of every following
  * sigma-vector.  If out is not NULL it receives, for classes 0..3,
  * {milliseconds, launches, work} (12 doubles; work in algorithmic flops for
