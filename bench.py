@@ -127,6 +127,8 @@ def timed_sigma(op, hip, dX, dW, nvec, prec, steps, warmup):
 KERNEL_DESC = {
     "int": "gemm_kernel<%s,*,tag=1> (virtual-index coupling contractions with the (vv|ov) block: "
            "down + up, mean per launch)",
+    "csf": "down_kernel, up_kernel<%s> (virtual-index coupling contractions on CSF vectors: down + up, "
+           "mean per launch)",
     "df": "gemm_kernel<%s,128,128,*,tag=1> (DF coupling contractions over naux: down + up, mean per launch)",
 }
 
@@ -134,7 +136,8 @@ KERNEL_DESC = {
 def roofline_of(prof, prec, workload, form):
     ms, launches, flops = prof["coupling_gemm"]
     achieved = flops / (ms * 1e-3) / 1e12
-    return {"kernel": KERNEL_DESC[form] % prec,
+    csf = form == "int" and prec != "bf16"  # nocc <= 32 in every workload here
+    return {"kernel": KERNEL_DESC["csf" if csf else form] % prec,
             "bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK[prec], "unit": "TFLOP/s",
             "frac": round(achieved / PEAK[prec], 4), "traffic": measured_traffic(prec, workload, form),
             "launches": int(launches), "avg_launch_ms": round(ms / max(launches, 1), 4),
