@@ -4,6 +4,7 @@
 
 #include <algorithm>
 
+#include "csf_index.hpp"
 #include "gemm.hpp"
 #include "kernels.hpp"
 

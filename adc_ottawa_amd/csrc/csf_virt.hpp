@@ -266,7 +266,7 @@ up_kernel(CsfGeo g, int vpb, int ug, const double* __restrict__ X, const double*
   typedef typename MT::Acc Acc;
   constexpr int PB = 8 / (int)sizeof(T);  // 16-pair blocks per chunk; lane li holds pairs PB*li ..
   constexpr int P = 16 * PB;
-  constexpr int KT = 8;                   // rows c per K tile
+  constexpr int KT = CSF_UP_ROWS;         // rows c per K tile
   constexpr int ARR = NL * KT * 128;
   typedef T tv __attribute__((ext_vector_type(PB)));
   __shared__ __attribute__((aligned(1024))) char s0[ARR];
@@ -288,7 +288,7 @@ up_kernel(CsfGeo g, int vpb, int ug, const double* __restrict__ X, const double*
   const bool live = row < rows;
   const int vec = live ? row / o : 0, k = live ? row - vec * o : 0;
   // the lane's next x1 value (rows past the last vector read zeros)
-  const char* xp = (const char*)(live ? X + g.ldx * (vec0 + vec) + k : zeros) + (int64_t)gq * o * 8;
+  const char* xp = (const char*)(live ? X + g.ldx * (vec0 + vec) + k : zeros) + (int64_t)csf_up_first(gq, v) * o * 8;
   const int64_t slab = (int64_t)v * 128;
   const char* src0 =
       (const char*)V + (diag ? (int64_t)2 * g.nch * o + (int64_t)ch * o : (int64_t)ch * 2 * o + (five ? o : 0)) * slab;
@@ -306,8 +306,8 @@ up_kernel(CsfGeo g, int vpb, int ug, const double* __restrict__ X, const double*
     for (int l = wave; l < o; l += nw) lds_copy(src, l * slab32 + c0 * 128, buf + l * 1024, lane16);
   };
   double xr[2];
-  const int64_t xhalf = (int64_t)o * 32, xstep = (int64_t)o * 64;
-  auto load_x = [&]() ADC2G_INLINE {  // (rows c past the last virtual are 2h2p entries, not used)
+  const int64_t xhalf = (int64_t)csf_up_half(v) * o * 8, xstep = (int64_t)o * KT * 8;
+  auto load_x = [&]() ADC2G_INLINE {  // (rows c past the last virtual are masked in operand)
     xr[0] = *(const double*)xp;
     xr[1] = *(const double*)(xp + xhalf);
     xp += xstep;
