@@ -128,40 +128,37 @@ void Handle::integral_block(bool virt, DevBuf<char>& out) {
 }
 
 // Operands of the CSF form in precision p, each rounded once from the FP64
-// blocks (which are kept only when the pair-tensor form has built them).
+// blocks.  The blocks stay: an operand that is first asked for later (FP32, the
+// pair tensors of BF16 and of the coupled preconditioner) then takes a pass over
+// them instead of a product over naux, and a new handle's first sigma-vector
+// does not run beside the release of 1 GB (o=16, v=200: creation with
+// keep_lowprec 82 -> 41 ms, first FP32 product without it 15 -> 3.4, first BF16
+// product 9.3 -> 4.0 ms).
 void Handle::build_csf(Prec p) {
   CsfSet& c = cs[p == Prec::F64 ? 0 : 1];
   if (c.ready) return;
-  DevBuf<char> tV, tO;
-  const char* V = is[0].V.get();
-  if (!is[0].ready) {
-    integral_block(true, tV);
-    V = tV.get();
-  }
+  build_integrals();
+  const double* V = (const double*)is[0].V.get();
   if (!cs_O.get()) {
-    const char* O = is[0].O.get();
-    if (!is[0].ready) {
-      integral_block(false, tO);
-      O = tO.get();
-    }
-    cs_O.alloc(csf_o_elems(dk));
-    launch_csf_build_o((const double*)O, dk, cs_O.get(), st);
     cs_zeros.alloc(csf_zeros(dk));
     HIP_CHECK(hipMemsetAsync(cs_zeros.get(), 0, sizeof(double) * csf_zeros(dk), st));
+    cs_O.alloc(csf_o_elems(dk));
+    launch_csf_build_o((const double*)is[0].O.get(), dk, cs_O.get(), st);
   }
   if (p == Prec::F64) {
     c.V.alloc(sizeof(double) * csf_v_elems<double>(dk));
-    launch_csf_build_v<double>((const double*)V, dk, (double*)c.V.get(), st);
+    launch_csf_build_v<double>(V, dk, (double*)c.V.get(), st);
   } else {
     c.V.alloc(sizeof(float) * csf_v_elems<float>(dk));
-    launch_csf_build_v<float>((const double*)V, dk, (float*)c.V.get(), st);
+    launch_csf_build_v<float>(V, dk, (float*)c.V.get(), st);
   }
   HIP_CHECK(hipStreamSynchronize(st));
   c.ready = true;
 }
 
-// Integral blocks of the pair-tensor form (BF16, and nocc > CSF_OMAX): Vt and
-// Ot are the same numbers in the layouts the up contractions read.
+// FP64 integral blocks, from which every other operand of the INT form is made.
+// Vt and Ot (nocc > CSF_OMAX: FP64 on pair tensors) are the same numbers in the
+// layouts the up contractions read.
 void Handle::build_integrals() {
   IntSet& s = is[0];
   if (s.ready) return;

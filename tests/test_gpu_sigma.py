@@ -215,3 +215,16 @@ def test_sigma_csf_edges(o, v, nvec, prec, tol):
         # one vector alone: another launch shape, the same numbers to rounding
         w = op.sigma(X[:, -1], precision=prec)
         assert np.abs(w - ref[:, -1]).max() < tol * np.abs(ref[:, -1]).max()
+
+
+# operands made at creation and on demand, in either order: the same numbers
+@pytest.mark.parametrize("order", [("fp64", "fp32", "bf16"), ("bf16", "fp32", "fp64")])
+def test_sigma_int_operands_on_demand(order):
+    print(f"[case] sigma int operands on demand {order}", flush=True)
+    sys = make_system(5, 37, 60, seed=9)
+    with lib.Operator.from_system(sys, coupling="int", keep_lowprec=True) as op:
+        X = np.random.default_rng(16).standard_normal((op.ndim, 6))
+        kept = {p: op.sigma(X, precision=p) for p in order}
+    with lib.Operator.from_system(sys, coupling="int") as op:
+        for p in order:
+            assert np.array_equal(op.sigma(X, precision=p), kept[p])
