@@ -72,10 +72,12 @@ struct CsfPlan {
   size_t down_bytes, occ_bytes, t2_bytes;
 };
 CsfPlan csf_plan(const DimsK& d, int nv);
+inline size_t ws_round(size_t bytes) { return (bytes + 255) / 256 * 256; }
 // The largest workspaces of passes of 1..nv vectors (fewer vectors can mean
 // more K splits, and more bytes).
 struct CsfBytes {
   size_t down = 0, occ = 0, t2 = 0;
+  size_t total() const { return ws_round(down) + ws_round(occ) + ws_round(t2); }
 };
 CsfBytes csf_workspace(const DimsK& d, int nv);
 

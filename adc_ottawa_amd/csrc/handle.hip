@@ -365,6 +365,12 @@ bool Handle::lowprec_ready(Prec p) const {
   return form == FORM_INT ? is[prec_index(p)].ready : (p == Prec::F64 ? fs[0].ready : fs[prec_index(p)].ready);
 }
 
+void Handle::csf_carve(const CsfBytes& b, char* w) {
+  ws_pdown = w;
+  ws_pocc = w + ws_round(b.down);
+  ws_pt2 = w + ws_round(b.down) + ws_round(b.occ);
+}
+
 // Vectors per pass that fit the caller's scratch: the workspace of the pass
 // (256-byte aligned regions) plus at least 32 MiB, or the per-vector
 // workspace if larger, for the GEMM split-K partials.
@@ -372,11 +378,9 @@ int Handle::scratch_chunk(Prec p) const {
   if (csf_form(p)) {
     // the partials of the CSF form hardly grow with the vectors; 24 vectors
     // keep the split-K partials of H11 x1 (about 1 MiB each) within the reserve
-    const size_t reserve = ((size_t)32 << 20) + 3 * 256;
-    for (int nc = 24; nc > 0; --nc) {
-      const CsfBytes b = csf_workspace(dk, nc);
-      if (b.down + b.occ + b.t2 + reserve <= scratch_bytes) return nc;
-    }
+    const size_t reserve = (size_t)32 << 20;
+    for (int nc = 24; nc > 0; --nc)
+      if (csf_workspace(dk, nc).total() + reserve <= scratch_bytes) return nc;
     return 0;
   }
   const size_t per = sigma_workspace_bytes(1, p) + 6 * 256;
@@ -417,14 +421,12 @@ void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nve
     char* q = scratch;
     auto carve = [&](size_t bytes) {
       char* r = q;
-      q += (bytes + 255) / 256 * 256;
+      q += ws_round(bytes);
       return (void*)r;
     };
     if (csf_form(p)) {
       const CsfBytes b = csf_workspace(dk, nc_max);
-      ws_pdown = carve(b.down);
-      ws_pocc = carve(b.occ);
-      ws_pt2 = carve(b.t2);
+      csf_carve(b, (char*)carve(b.total()));
     } else {
       ws_x1c = carve(n1 * nc_max * es);
       ws_zg = carve(n1 * n1 * nc_max * es);
@@ -446,12 +448,8 @@ void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nve
     gws.ext_size = 0;
     if (csf_form(p)) {
       const CsfBytes b = csf_workspace(dk, nc_max);
-      Pdown.alloc(b.down);
-      Pocc.alloc(b.occ);
-      Pt2.alloc(b.t2);
-      ws_pdown = Pdown.get();
-      ws_pocc = Pocc.get();
-      ws_pt2 = Pt2.get();
+      Pcsf.alloc(b.total());
+      csf_carve(b, Pcsf.get());
     } else {
       X1c.alloc(n1 * nc_max * es);
       ZG.alloc(n1 * n1 * nc_max * es);

@@ -68,7 +68,10 @@ struct Handle {
   DevBuf<char> Wup;         // W[P][vec][(c,k)] (accumulator type: FP64, or FP32 for FP32/BF16)
   DevBuf<char> WupT;        // W transposed, [(vec,c,k)][P], GEMM precision
   DevBuf<char> ZG;          // Z then G, in the chunk's GEMM precision
-  DevBuf<char> Pdown, Pocc, Pt2;  // 1h1p partials and t2 copy of the CSF form
+  // 1h1p partials and t2 copy of the CSF form, in one buffer (three took 0.28 ms
+  // more to grow from 2 to 20 vectors at o=5, v=36, where the product takes 0.06)
+  DevBuf<char> Pcsf;
+  void csf_carve(const CsfBytes& b, char* w);
   // workspaces of the current sigma pass: the buffers above, or regions of
   // a caller's scratch (sigma with `scratch` set allocates nothing)
   void *ws_x1c = nullptr, *ws_x1t = nullptr, *ws_zg = nullptr, *ws_yvv = nullptr, *ws_yoo = nullptr,
