@@ -532,9 +532,8 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   // two workgroups per CU are in flight, each with three slabs or more.  The
   // split orders the sums.  From 2 to 24 slabs its time at small sizes is the
   // same to 1 us, so three was taken, in even numbers of workgroups, as the
-  // order under which solver runs that amplify the last bit (iterations to
-  // 1e-7 of the uncoupled-guess block Davidson; partially re-orthogonalised
-  // Lanczos past the loss of orthogonality) stay closest to the NumPy oracle
+  // order under which a solver run that amplifies the last bit (iterations to
+  // 1e-7 of the uncoupled-guess block Davidson) stays closest to the NumPy oracle
   const int nb = (v + 15) / 16;
   p.dns = (nb + 12) / 13;
   p.dnb = (nb + p.dns - 1) / p.dns;

@@ -584,13 +584,8 @@ void lanczos_run(Handle& H, const adc2g_lanczos_params& p, const double* q0_h, d
     upper_inverse(b, R1.data(), Ri.data());
     upload_small(Ri);
     gemm_nn(H, n, b, b, U.get(), n, small.get(), b, X2.get(), n, 1.0, 0.0);
-    // two Cholesky QR passes: U = X2 R2^-1, Q_{j+1} = U R3^-1
-    double* Qn = L.get() + (size_t)n * b * (j + 1);
-    Qn_cur = Qn;
-    for (int pass = 0; pass < 2; ++pass) {
-      const double* src = pass == 0 ? X2.get() : U.get();
-      double* dst = pass == 0 ? U.get() : Qn;
-      std::vector<double>& Rk = pass == 0 ? R2 : R3;
+    // one Cholesky QR pass: src = dst Rk
+    auto cholqr = [&](const double* src, double* dst, std::vector<double>& Rk) {
       gram_to_host(src, G);
       if (!cholesky_upper(b, G.data(), Rk.data()))
         throw Error(ADC2G_EBREAK, "block Lanczos: the residual block of cycle " + std::to_string(j + 1) +
@@ -598,7 +593,12 @@ void lanczos_run(Handle& H, const adc2g_lanczos_params& p, const double* q0_h, d
       upper_inverse(b, Rk.data(), Ri.data());
       upload_small(Ri);
       gemm_nn(H, n, b, b, src, n, small.get(), b, dst, n, 1.0, 0.0);
-    }
+    };
+    // two of them: U = X2 R2^-1, Q_{j+1} = U R3^-1
+    double* Qn = L.get() + (size_t)n * b * (j + 1);
+    Qn_cur = Qn;
+    cholqr(X2.get(), U.get(), R2);
+    cholqr(U.get(), Qn, R3);
     // B_j = R3 R2 R1
     upper_mul(b, R2.data(), R1.data(), W1.data());
     upper_mul(b, R3.data(), W1.data(), Bprev.data());
@@ -609,6 +609,25 @@ void lanczos_run(Handle& H, const adc2g_lanczos_params& p, const double* q0_h, d
       B_all.push_back(Bprev);
       const int jj = j + 1;  // the reference's 1-based cycle
       bool lro = false;
+      // A residual block at the rounding of H Q_j (an invariant subspace: the
+      // start block of eigenvectors that a guess over the whole space gives, or
+      // an exhausted Krylov space) leaves in Q_{j+1} components of order one
+      // along every stored block, and taking them out of orthonormal columns
+      // leaves columns that are not.  Such a block is made orthogonal to all
+      // stored blocks and orthonormal, twice; B_j stays at the rounding of T.
+      // Above the limit the components are below sqrt(eps), and what their
+      // removal changes in the products of the columns is below eps.
+      double scale2 = 0.0;
+      for (int i = 0; i < b * b; ++i)
+        scale2 += A[i] * A[i] + Bprev[i] * Bprev[i] + (jj > 1 ? B_all[jj - 2][i] * B_all[jj - 2][i] : 0.0);
+      const auto sb = svd_ends(Bprev);
+      const bool fresh = sb.second <= orthlim * std::sqrt(scale2);
+      if (fresh)
+        for (int pass = 0; pass < 2; ++pass) {
+          double* src = pass == 0 ? Qn : U.get();
+          for (int k = 0; k <= j; ++k) project_out(L.get() + (size_t)n * b * k, src);
+          cholqr(src, pass == 0 ? U.get() : Qn, R1);
+        }
       if (jj > 1 && jj < m) {
         // update_omega (:1530-1639)
         if (jj == 2) {
@@ -620,7 +639,6 @@ void lanczos_run(Handle& H, const adc2g_lanczos_params& p, const double* q0_h, d
           OM(1, 2) = OM(2, 1) = om_eps / s2.second;
         }
         anorm[jj] = svd_ends(A_all[jj - 1]).first;
-        const auto sb = svd_ends(B_all[jj - 1]);
         bnorm[jj] = sb.first;
         const double inv = 1.0 / sb.second;
         OM(jj, jj + 1) = OM(jj + 1, jj) = OM(jj + 1, jj + 1) = om_eps;
@@ -630,7 +648,11 @@ void lanczos_run(Handle& H, const adc2g_lanczos_params& p, const double* q0_h, d
           x += bnorm[jj] * OM(jj - 1, k) + (anorm[jj] + anorm[k]) * OM(jj, k);
           OM(jj + 1, k) = OM(k, jj + 1) = inv * x;
         }
-        if (p.orthotype == 2) {
+        if (fresh) {
+          for (int k = 1; k <= jj; ++k) OM(jj + 1, k) = OM(k, jj + 1) = om_eps;
+          ivs.clear();
+          l2nd = false;
+        } else if (p.orthotype == 2) {
           lro = mpro(jj);
         } else {
           for (int k = 1; k < jj; ++k)
@@ -649,7 +671,7 @@ void lanczos_run(Handle& H, const adc2g_lanczos_params& p, const double* q0_h, d
           for (int k = 1; k <= jj; ++k) OM(jj + 1, k) = OM(jj, k) = om_eps;
         }
       }
-      if (p.orthotype == 1) {
+      if (p.orthotype == 1 && !fresh) {
         // localro (:1430-1470): Q_{j+1} against Q_j, normalised
         project_out(Pw.get(), Qn);
         normalise_cols(Qn);

@@ -567,7 +567,10 @@ int32_t adc2g_power(adc2g_handle* h, int32_t subdim, int32_t maxit, double thrsh
  * re-orthogonalisation (mpro, mpro_mgs, lowerbound, upperbound, :1710-1890):
  * the same omega recurrence, Q_{j+1} alone against the intervals of stored
  * blocks around the estimates that reach sqrt(eps), the widened intervals once
- * more in the next cycle, no localro.
+ * more in the next cycle, no localro.  With either, a residual block at the
+ * rounding of H Q_j (an invariant subspace; the reference goes on with a
+ * Q_{j+1} that is not orthonormal) is made orthonormal and orthogonal to all
+ * stored blocks, and npro does not count it.
  *   U = H Q_j - Q_{j-1} B_{j-1}^T,  A_j = Q_j^T U,  R = U - Q_j A_j = Q_{j+1} B_j
  * with B_j upper triangular.  The reference factors R with dgeqrf/dorgqr; here a
  * shifted Cholesky QR with two refinement passes gives the factor with a

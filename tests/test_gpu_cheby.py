@@ -112,6 +112,23 @@ def test_spectral_bounds_davlanc(form):
     assert abs(hi - lam[-1]) < 1e-7 * scale
 
 
+@pytest.mark.parametrize("o,v,naux", [(3, 8, 10), (2, 6, 12), (3, 10, 14)])
+@pytest.mark.parametrize("seed", range(6))
+def test_spectral_bounds_davlanc_whole_space_guess(o, v, naux, seed):
+    """Up to 800 configurations the guess subspace is the whole space and the
+    Lanczos start block two eigenvectors, so that its first residual is
+    rounding: the bounds are the extreme eigenvalues for every system.  (A bound
+    above the spectrum by several Eh was the rule on half of them.)"""
+    print(f"[case] spectral bounds o={o} v={v} naux={naux} seed={seed}", flush=True)
+    sys = make_system(o, v, naux, seed=seed)
+    lam = np.linalg.eigvalsh(elements.build_blocks(sys, apply_minc=False).dense())
+    with lib.Operator.from_system(sys) as op:
+        lo, hi = op.spectral_bounds(ncycles=min(100, lam.size // 2))
+    scale = np.abs(lam).max()
+    assert abs(lo - lam[0]) < 1e-9 * scale      # Davidson to 1e-8
+    assert abs(hi - lam[-1]) < 1e-11 * scale    # up to 200 Lanczos vectors, converged: rounding
+
+
 @pytest.mark.parametrize("form", FORMS)
 def test_power_method_vs_oracle(form):
     """power_method with a 20-IS guess (about 200 iterations): the oracle's

@@ -160,6 +160,28 @@ def test_lanczos_modified_partial_reorthogonalisation_vs_oracle(form):
     assert (np.abs(ev - lam[-1]) < 1e-6).sum() == 1
 
 
+@pytest.mark.parametrize("orthotype", [1, 2])
+@pytest.mark.parametrize("b", [1, 2, 3])
+def test_lanczos_invariant_start_block(orthotype, b):
+    """A start block of eigenvectors: the first residual is rounding, and the
+    recurrence goes on in the rest of the space.  The stored vectors stay
+    orthogonal to the sqrt(eps) that partial re-orthogonalisation keeps, the
+    start's eigenvalues are among those of T, and the top one is the matrix's,
+    once."""
+    print(f"[case] lanczos invariant start o=3 v=8 b={b} orthotype={orthotype}", flush=True)
+    sys = make_system(3, 8, 10, seed=3)
+    H = elements.build_blocks(sys, apply_minc=False).dense()
+    lam, U = np.linalg.eigh(H)
+    q0 = np.ascontiguousarray(U[:, 100:100 + b])
+    with lib.Operator.from_system(sys) as op:
+        ev, _, st = op.block_lanczos(q0, 180 // b, orthotype=orthotype, check_orth=True)
+    scale = np.abs(lam).max()
+    assert st["orth_loss"] < 1e-7
+    assert np.abs(ev[:, None] - lam[None, 100:100 + b]).min(axis=0).max() < 1e-11 * scale
+    assert abs(ev[-1] - lam[-1]) < 1e-11 * scale
+    assert (np.abs(ev - lam[-1]) < 1e-6).sum() == 1
+
+
 @pytest.mark.parametrize("kind,b", [(8, 2), (8, 4), (9, 3)])
 def test_lanczos_guess_vs_oracle(kind, b):
     """init_vec_doublesubspace (8) / init_vec_singlesubspace (9) with a
