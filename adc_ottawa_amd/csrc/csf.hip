@@ -546,8 +546,12 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   p.ds = (int)std::max<int64_t>(1, std::min<int64_t>(tiles / 6 * 2, 512 / ((int64_t)p.dg * p.dns)));
   // one pass for both directions where the rows fit two 16-row blocks and a
   // slab's columns the registers, and every workgroup has work for two rounds
-  // (o=16, v=200: one vector 0.29 ms against 0.26 + 0.27 in two passes, two
-  // vectors 0.49 against 0.33 + 0.30; o=5, v=36, 83 chunks: 17 us against 15)
+  // also with the fewer chunks of FP32, that is from v = 128 on (o=16, v=200:
+  // one vector 0.29 ms against 0.26 + 0.27 in two passes, two vectors 0.49
+  // against 0.33 + 0.30; o=5, v=36, 83 chunks: 17 us against 15).  A whole
+  // product of one vector, one pass against two, FP64 and FP32: o=16, v=128 147
+  // against 220 and 134 against 148 us, o=3, v=128 55 against 57 and 50 against
+  // 51; o=5, v=112 70 against 65 and 66 against 60
   const int items = 2 * g4.nch + g4.nchd;
   p.thin = (o <= 16 && rows <= 32 && v <= 208 && items >= 512) ? 256 : 0;
   p.down_bytes = (size_t)std::max(p.ds, p.thin) * rows * v * sizeof(double);

@@ -758,9 +758,9 @@ void thin_launch(const CsfGeo& g, const CsfPlan& p, const double* X, const doubl
                  double* W, typename Mma<T>::Acc* part, hipStream_t st) {
   const dim3 grid((unsigned)p.thin), blk(256);
   const int nb = (g.v + 15) / 16;
-  if (nb <= 4)
-    hipLaunchKernelGGL((thin_kernel<T, 4, 2, TM>), grid, blk, 0, st, g, X, T2, zeros, V, W, part);
-  else if (nb <= 8)
+  // thin plans start at v = 128 (eight blocks): two vectors, o = 16, FP64 there
+  // 237 us, with the parts of 13 blocks 255
+  if (nb <= 8)
     hipLaunchKernelGGL((thin_kernel<T, 8, 2, TM>), grid, blk, 0, st, g, X, T2, zeros, V, W, part);
   else
     hipLaunchKernelGGL((thin_kernel<T, 13, 4, TM>), grid, blk, 0, st, g, X, T2, zeros, V, W, part);
