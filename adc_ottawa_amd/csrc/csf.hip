@@ -529,11 +529,11 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   const int rows = nv * o, waves = (rows + 15) / 16;
   // down: rows in groups of dw waves (4, or fewer when there are no more),
   // columns in equal splits of at most 13 blocks of 16, K split so that about
-  // two workgroups per CU are in flight, each with three slabs or more.  The
-  // split orders the sums.  From 2 to 24 slabs its time at small sizes is the
-  // same to 1 us, so three was taken, in even numbers of workgroups, as the
-  // order under which a solver run that amplifies the last bit (iterations to
-  // 1e-7 of the uncoupled-guess block Davidson) stays closest to the NumPy oracle
+  // two workgroups per CU are in flight, each with three slabs or more: with
+  // fewer the sum over the splits grows, with more the chain of a workgroup does
+  // (whole product with at least 1, 2, 3, 4, 8 slabs, FP64: o=4, v=24, 20 vectors
+  // 40.6, 41.0, 42.3, 43.2, 47.8 us; o=5, v=36, 20 vectors 53.5, 50.3, 50.6, 51.9,
+  // 56.4; o=8, v=60, one vector 54.4, 53.6, 52.1, 52.6, 57.3)
   const int nb = (v + 15) / 16;
   p.dns = (nb + 12) / 13;
   p.dnb = (nb + p.dns - 1) / p.dns;
@@ -543,7 +543,7 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   p.dg = (waves + p.dw - 1) / p.dw;
   const CsfGeo g8 = csf_geo<double>(d, nv, 0, 0), g4 = csf_geo<float>(d, nv, 0, 0);
   const int64_t tiles = std::min((int64_t)(2 * g8.nch + g8.nchd), (int64_t)(2 * g4.nch + g4.nchd)) * o;
-  p.ds = (int)std::max<int64_t>(1, std::min<int64_t>(tiles / 6 * 2, 512 / ((int64_t)p.dg * p.dns)));
+  p.ds = (int)std::max<int64_t>(1, std::min<int64_t>(tiles / 3, 512 / ((int64_t)p.dg * p.dns)));
   // one pass for both directions where the rows fit two 16-row blocks and a
   // slab's columns the registers, and every workgroup has work for two rounds
   // also with the fewer chunks of FP32, that is from v = 128 on (o=16, v=200:

@@ -126,7 +126,12 @@ def test_water_subdiag_guess_vs_oracle(water, precon):
 
 def test_water_adc1_guess_vs_oracle(water):
     """Initial vectors given by the caller (initvec_adc1): the ADC(1)
-    eigenvectors, from the first-order ph-ph block, zero on the 2h2p part."""
+    eigenvectors, from the first-order ph-ph block, zero on the 2h2p part.  The
+    number of iterations from these amplifies the last bit of the sums: 48 runs of
+    the oracle whose products were perturbed by 1e-16 of their largest element
+    took 257 to 345, mean 317, standard deviation 20 (the same perturbation moves
+    the runs from other guesses above, of about 100 iterations, by one at most).
+    Bar: five deviations about that mean."""
     sys, blk, w, op = water
     b1 = elements.build_blocks(sys, second_order=False)
     _, U = np.linalg.eigh(b1.H11)
@@ -135,10 +140,12 @@ def test_water_adc1_guess_vs_oracle(water):
     ev, X, st = op.davidson(5, maxvec=40, tol=1e-7, precon="dpr", guess=g, maxiter=500)
     print("ADC(1) guess: per-root |E - E_arpack|", np.abs(ev - w), "iterations", st["niter"])
     assert np.abs(ev - w).max() < 1e-8
+    assert residual_norms(blk.sigma, ev, X).max() < 1e-7 * 1.01
     ref = odav.davidson(blk.sigma, blk.diag(), 5, blocksize=5, maxvec=40, tol=1e-7, precon=1,
                         deflate=False, maxiter=500, guess=g)
     assert np.abs(ref["eigval"] - ev).max() < 1e-8
-    assert abs(ref["niter"] - st["niter"]) <= 3
+    for niter in (ref["niter"], st["niter"]):
+        assert abs(niter - 317) <= 5 * 20
 
 
 def test_guess_errors(water):
