@@ -371,22 +371,23 @@ void Handle::csf_carve(const CsfBytes& b, char* w) {
   ws_pt2 = w + ws_round(b.down) + ws_round(b.occ);
 }
 
-// Vectors per pass that fit the caller's scratch: the workspace of the pass
-// (256-byte aligned regions) plus at least 32 MiB, or the per-vector
-// workspace if larger, for the GEMM split-K partials.
-int Handle::scratch_chunk(Prec p) const {
-  if (csf_form(p)) {
-    // the partials of the CSF form hardly grow with the vectors; 24 vectors
-    // keep the split-K partials of H11 x1 (about 1 MiB each) within the reserve
-    const size_t reserve = (size_t)32 << 20;
-    for (int nc = 24; nc > 0; --nc)
-      if (csf_workspace(dk, nc).total() + reserve <= scratch_bytes) return nc;
-    return 0;
-  }
+// Scratch of a pass of nc vectors: its workspace (256-byte aligned regions) and
+// the GEMM split-K partials, 32 MiB or, on pair tensors, the workspace of one
+// vector where that is larger.
+size_t Handle::scratch_need(int nc, Prec p) const {
+  const size_t partials = (size_t)32 << 20;
+  if (csf_form(p)) return csf_workspace(dk, nc).total() + partials;
   const size_t per = sigma_workspace_bytes(1, p) + 6 * 256;
-  const size_t reserve = std::max<size_t>((size_t)32 << 20, per);
-  if (scratch_bytes < per + reserve) return 0;
-  return (int)std::min<size_t>((size_t)chunk, (scratch_bytes - reserve) / per);
+  return nc * per + std::max(partials, per);
+}
+
+// Vectors per pass that fit the caller's scratch.  The partials of the CSF form
+// hardly grow with the vectors; 24 keep those of H11 x1 (about 1 MiB a vector,
+// whatever n1) within their share.
+int Handle::scratch_chunk(Prec p) const {
+  int nc = csf_form(p) ? 24 : chunk;
+  while (nc > 0 && scratch_need(nc, p) > scratch_bytes) --nc;
+  return nc;
 }
 
 // W = H X for nvec columns (device pointers, ld = ldx / ldw), in chunks of at
@@ -416,8 +417,9 @@ void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nve
     ARG_CHECK(lowprec_ready(p), "the operands of this precision are not resident (create the handle with "
                                 "keep_lowprec = 1 or run one sigma-vector of this precision first)");
     nc_max = std::min(nvec, scratch_chunk(p));
-    ARG_CHECK(nc_max >= 1, "one vector needs " + std::to_string(sigma_workspace_bytes(1, p)) +
-                               " bytes of scratch; the scratch holds " + std::to_string(scratch_bytes));
+    if (nc_max < 1)
+      throw Error(ADC2G_ENOMEM, "one vector needs " + std::to_string(scratch_need(1, p)) +
+                                    " bytes of scratch; the scratch holds " + std::to_string(scratch_bytes));
     char* q = scratch;
     auto carve = [&](size_t bytes) {
       char* r = q;

@@ -79,6 +79,7 @@ struct Handle {
   char* scratch = nullptr;
   size_t scratch_bytes = 0;
   bool lowprec_ready(Prec p) const;
+  size_t scratch_need(int nc, Prec p) const;
   int scratch_chunk(Prec p) const;
   GemmWorkspace gws;
   DevBuf<double> skinny_ws;  // per-block partials of the tall-skinny products

@@ -1,7 +1,7 @@
 """adc2g_sigma_device_noalloc (the sigma-vector that allocates nothing, all
 workspaces in the library's static scratch) against adc2g_sigma_device on the
 same device buffers, through the C ABI: two calls in a row, the second with
-fewer vectors; FP64 to 1e-12 relative, FP32/BF16 to 1e-5 of the largest
+fewer vectors, and calls of several passes; FP64 to 1e-12 relative, FP32/BF16 to 1e-5 of the largest
 element (the passes differ only in how many vectors share a GEMM, which can
 change split-K summation orders).  Error paths: a CVS view and a precision
 whose operands are not resident are rejected without work."""
@@ -95,7 +95,7 @@ def test_noalloc_benzene_and_errors():
         hip.free(dX)
         hip.free(dW)
         assert rc == 10
-        # FP64: two vectors per pass at this size; 5 vectors then 2
+        # FP64: one pass each, the second, of fewer vectors, by another kernel
         for nvec in (5, 2):
             X = rng.standard_normal((op.ndim, nvec))
             A, B = run_pair(op, hip, X, "fp64")
@@ -111,3 +111,45 @@ def test_noalloc_benzene_and_errors():
             hip.free(dX)
             hip.free(dW)
             assert rc == 10
+
+
+def test_noalloc_benzene_passes():
+    """FP64 and FP32 take up to 24 vectors per pass: 25 and 49 vectors end with a
+    pass of one, whose kernel and partial sums are other ones than those the
+    regions were sized by; adc2g_sigma_device takes all of them in one pass."""
+    sz = SIZES["benzene"]
+    print(f"[case] noalloc benzene passes {sz}", flush=True)
+    hip = Hip()
+    sys_ = make_system(seed=0, **sz)
+    with lib.Operator.from_system(sys_, coupling="int", keep_lowprec=True) as op:
+        X = np.random.default_rng(8).standard_normal((op.ndim, 25), dtype=np.float32).astype(np.float64)
+        X2 = np.hstack([X, 0.5 * X[:, :24] - X[:, 1:]])
+        for prec, tol, Y in (("fp64", 1e-12, X), ("fp32", 1e-5, X), ("fp64", 1e-12, X2)):
+            A, B = run_pair(op, hip, Y, prec)
+            # every vector on its own scale
+            err = (np.abs(A - B).max(axis=0) / np.abs(A).max(axis=0)).max()
+            print(f"{prec} nvec {Y.shape[1]}: max |W_noalloc - W| / max |W| = {err:.2e}", flush=True)
+            assert err <= tol
+
+
+def test_noalloc_does_not_fit():
+    """DF form in FP64 at o=16, v=200: one vector's pair tensor and factor
+    products exceed the scratch.  ADC2G_ENOMEM, and W is left alone."""
+    print("[case] noalloc does not fit", flush=True)
+    hip = Hip()
+    L = lib.load()
+    with lib.Operator.from_system(make_system(seed=0, **SIZES["benzene"]), coupling="df") as op:
+        X = np.ones((op.ndim, 1))
+        W = np.full((op.ndim, 1), 7.0)
+        dX, dW = hip.malloc(X.nbytes), hip.malloc(W.nbytes)
+        try:
+            hip.h2d(dX, X)
+            hip.h2d(dW, W)
+            rc = L.adc2g_sigma_device_noalloc(op.handle, 1, C.c_void_p(dX), C.c_void_p(dW), lib.PREC["fp64"], None)
+            hip.sync()
+            hip.d2h(W, dW)
+        finally:
+            hip.free(dX)
+            hip.free(dW)
+    assert rc == 14
+    assert np.all(W == 7.0)
