@@ -14,7 +14,7 @@ import pytest
 
 from adc_ottawa_amd import lib
 from adc_ottawa_amd.synth import SIZES, make_system
-from oracle import adcx, elements
+from oracle import adcx, dfsigma, elements
 
 pytestmark = pytest.mark.gpu
 
@@ -51,6 +51,26 @@ def test_adcx_sigma_and_diagonal(form, o, v, naux, seed):
     assert np.abs(d_x - np.diag(H)).max() < 1e-12 * np.abs(np.diag(H)).max()
     assert np.abs(W_back - W_s).max() == 0.0 and np.abs(d_back - d_s).max() < 1e-14 * np.abs(d_s).max()
     assert np.abs(W_x - W_s).max() > 1e-6 * np.abs(ref).max()       # the block is not trivially zero
+
+
+# runs of pairs that leave a remainder in the tiled ring layouts (16 virtuals a run
+# at few occupied orbitals, one at 64), the element-wise layouts beyond 64, padded
+# and whole rows of the ladder products, and (19 vectors) a second chunk of vectors
+@pytest.mark.parametrize("o,v,nvec", [(2, 2, 1), (3, 20, 19), (4, 37, 2), (2, 33, 17), (9, 18, 3), (33, 5, 2),
+                                      (64, 2, 2), (65, 2, 2), (66, 4, 2)])
+def test_adcx_sigma_edges(o, v, nvec):
+    print(f"[case] adcx sigma edges o={o} v={v} nvec={nvec}", flush=True)
+    sys_ = make_system(o, v, 12, seed=o + v)
+    df = dfsigma.DF(sys_)
+    n1 = df.n1
+    X = np.random.default_rng(17).standard_normal((n1 + df.D2.size, nvec))
+    ref = df.sigma(X)
+    ref[n1:] += adcx.block22(sys_, X[n1:])
+    with lib.Operator.from_system(sys_) as op:
+        op.set_adc2x(True)
+        W = op.sigma(X)
+    for rows in (slice(0, n1), slice(n1, None)):
+        assert np.abs(W[rows] - ref[rows]).max() < 1e-11 * np.abs(ref[rows]).max()
 
 
 def test_adcx_davidson_roots():
