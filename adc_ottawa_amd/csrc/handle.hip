@@ -5,11 +5,13 @@
 // get_offdiag_adc2_save_omp, source/adclib/get_matrix.f90:705-1186) and then
 // multiplies with it (hxvec_incore, source/eigen/block_davidson.f90:844-883).
 // Here only the dense ph-ph block (n1 x n1) is built; the 1h1p<->2h2p
-// coupling is applied on the fly as MFMA contractions of the pair tensor of
-// the 2h2p amplitudes, either with the density-fitting factors (DF form, sums
-// over naux) or with the (vv|ov) and (oo|ov) blocks assembled once from them
-// (INT form, sums over v and o), and the 2h2p-2h2p block (diagonal,
-// adc_ph.f90:1090-1096) is fused into the pair-to-CSF projection.
+// coupling is applied on the fly as MFMA contractions, either with the
+// density-fitting factors (DF form, sums over naux) or with the (vv|ov) and
+// (oo|ov) blocks assembled once from them (INT form, sums over v and o).  The
+// INT form takes the CSF vectors as they are in FP64 and FP32 up to CSF_OMAX
+// occupied orbitals, and the pair tensor of the 2h2p amplitudes otherwise, as
+// the DF form does.  The 2h2p-2h2p block (diagonal, adc_ph.f90:1090-1096) is
+// fused into the pair-to-CSF projection, or into the occupied term of the CSFs.
 #include "handle.hpp"
 
 #include <algorithm>
@@ -81,8 +83,10 @@ void Handle::create(int o, int v, int naux, const double* eps_h, const double* B
   build_phph(dB.get(), nbas);
   HIP_CHECK(hipStreamSynchronize(st));
   // coupling form: the integral blocks need (v + o)/naux of the flops of the
-  // factor contractions, for v*v*n1 + o*o*n1 stored elements (twice: both
-  // operand layouts) per precision
+  // factor contractions, for v*v*n1 + o*o*n1 stored elements per precision,
+  // twice: both operand layouts, or the blocks and the operand on CSF vectors
+  // (FP32 there has the operand only and is counted as two).  The line at 0.6 is
+  // that of the pair tensors; on CSF vectors INT pays further up
   size_t need = integral_bytes(Prec::F64);
   if (opts.keep_lowprec) need += integral_bytes(Prec::F32) + integral_bytes(Prec::BF16);
   const size_t int_budget = (size_t)96 << 30;
@@ -391,9 +395,10 @@ int Handle::scratch_chunk(Prec p) const {
 }
 
 // W = H X for nvec columns (device pointers, ld = ldx / ldw), in chunks of at
-// most `chunk` vectors.  The 1h1p-1h1p block H11 x1 is always FP64; every
-// coupling contraction runs in the GEMM precision p (FP32 accumulation for
-// FP32/BF16), the 2h2p diagonal in FP64 inside the pair->CSF projection.
+// most `chunk` vectors, 64 on CSF vectors.  The 1h1p-1h1p block H11 x1 and the
+// 2h2p diagonal are always FP64; the coupling contractions run in the GEMM
+// precision p (FP32 accumulation for FP32/BF16), but for the occupied terms on
+// CSF vectors, which are FP64.
 void Handle::sigma(const double* X, int64_t ldx, double* W, int64_t ldw, int nvec, Prec p, hipStream_t s) {
   ARG_CHECK(ldx >= d.ndim && ldw >= d.ndim, "leading dimensions must be >= ndim");
   if (nvec <= 0) return;
