@@ -572,15 +572,17 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   p.nt = nb;
   // occupied: slices of the sets so that the workgroups come in whole rounds
   // of two per CU (three with one vector each: their registers); the fewest
-  // slices among equals
+  // slices among equals, at most 32 and, where those leave the round unfilled,
+  // 64 (one vector, FP32: o=32, v=33 167 -> 136 us, o=30, v=60 182 -> 155; pair
+  // tensors took 138 and 176)
   const int vgl = csf_occ_vectors(o, nv), vgs = (nv + vgl - 1) / vgl;
   const int64_t slots = o <= 16 && vgl == 1 ? 768 : 512;
   const int64_t wgs = (int64_t)(nb * (nb + 1) / 2 + 3) / 4 * vgs;
   double beff = 0.0;
   p.sl = 1;
-  for (int sl = 1; sl <= 32 && sl <= (int)(2 * d.npo + o + 3) / 4; ++sl) {
+  for (int sl = 1; sl <= 64 && sl <= (int)(2 * d.npo + o + 3) / 4; ++sl) {
     const int64_t n = wgs * sl;
-    if (n > 2048 && sl > 1) break;
+    if ((n > 2048 && sl > 1) || (n > slots && sl > 32)) break;
     const double eff = (double)n / (double)((n + slots - 1) / slots * slots);
     if (eff > 1.03 * beff) {
       beff = eff;
