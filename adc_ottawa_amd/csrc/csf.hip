@@ -555,12 +555,15 @@ CsfPlan csf_plan(const DimsK& d, int nv) {
   const int items = 2 * g4.nch + g4.nchd;
   p.thin = (o <= 16 && rows <= 32 && v <= 208 && items >= 512) ? 256 : 0;
   p.down_bytes = (size_t)std::max(p.ds, p.thin) * rows * v * sizeof(double);
-  // up: whole vectors per workgroup, the number of waves that pads least
+  // up: whole vectors per workgroup, the number of waves that pads least; no
+  // more vectors than leave each CU a workgroup (64 vectors, FP64: o=2, v=4 53 ->
+  // 29 us, o=2, v=16 58 -> 36; pair tensors took 53 and 67)
   const int wmax = o <= 16 ? 8 : 4;
+  const int groups = std::min(nv, std::max(1, 256 / (2 * g8.nch + g8.nchd))), cap = (nv + groups - 1) / groups;
   double best = 1e300;
   for (int w : {4, 8, 6, 2, 1}) {
     if (w > wmax || 16 * w < o) continue;
-    const int vpb = std::min(nv, 16 * w / o), grp = (nv + vpb - 1) / vpb;
+    const int vpb = std::min(cap, 16 * w / o), grp = (nv + vpb - 1) / vpb;
     const double cost = (double)grp * w * (w == 6 ? 1.05 : 1.0);
     if (cost < best) {
       best = cost;

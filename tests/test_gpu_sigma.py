@@ -199,7 +199,9 @@ CSF_CASES = [(2, 2, 1), (2, 33, 65), (3, 17, 5), (15, 18, 9), (16, 32, 5), (17, 
              # the first virtual count of that pass, whose slabs come in parts of their own
              (2, 128, 8), (3, 128, 10), (16, 128, 2), (15, 128, 1),
              # few tiles of virtuals and many occupied pairs: more slices of these
-             (32, 33, 1), (27, 18, 2), (17, 20, 6)]
+             (32, 33, 1), (27, 18, 2), (17, 20, 6),
+             # few chunks of pairs and many vectors: fewer of them per workgroup than its rows hold
+             (2, 5, 64), (3, 9, 23), (16, 17, 40)]
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
