@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(CP_THREADS) cp_unit_pairs_kernel(int o, int v,
   }
 }
 
-// The same tensor with one workgroup per c and CP_VECS vectors: every V value
+// The same tensor with one workgroup per c and `vecs` vectors: every V value
 // their rows read -- R[x] = V[c][a'][x] for x = (b,l) and S[b][m] =
 // V[b][a'][c o + m] -- is staged in LDS once per a' by coalesced loads (the
 // per-row kernel above gathers the l = k' and b-strided terms one element per
@@ -181,17 +181,25 @@ __global__ void __launch_bounds__(CP_THREADS) cp_unit_pairs_kernel(int o, int v,
 //
 // A row with k != k' and c != a' is zero but for l = k' and b = a'.  A thread
 // takes W consecutive elements (one 16-byte store; W = 1 where a row is not a
-// multiple of that) and computes at most the one with l = k'; the o x o
-// elements with b = a' follow in a second pass, since in the first a wave that
-// meets one would run all its elements and wait for their integrals in turn.
-// Then the writes bound it: o = 16, v = 200, 64 vectors in BF16 (1.3 GB) take
-// 0.47 ms (2.8 TB/s); one element at a time with every condition and one vector
-// per workgroup took 1.14 ms.
-constexpr int CP_VECS = 4;  // 3200 workgroups at o = 16, v = 200, 64 vectors
+// multiple of that, or l takes fewer values) and computes at most the one with
+// l = k'; the o x o elements with b = a' follow in a second pass, since in the
+// first a wave that meets one would run all its elements and wait for their
+// integrals in turn.  Then the writes bound it: o = 16, v = 200, 64 vectors in BF16
+// (1.3 GB) take 0.43 ms (3.1 TB/s); one element at a time with every condition and
+// one vector per workgroup took 1.14 ms.
+//
+// Consecutive vectors share a', and with it what is staged; but one c has it too,
+// and its vectors, formed element by element, follow one another on one
+// workgroup.  That is two vectors, and four below eight occupied orbitals, where
+// the staging is the longer part (a whole A0 in BF16 with 4, 2, 1 vectors: o=16,
+// v=200 79.0, 77.0, 79.2 ms; o=24, v=130 85.9, 78.7, 77.3; o=40, v=20 4.4, 3.4,
+// 2.8, where one vector and element at a time took 3.5; o=8, v=250 23.9, 24.6,
+// 26.2; o=4, v=400 20.3, 20.8, 22.0).
 constexpr int UP_THREADS = 512;  // two workgroups per CU by their LDS: four waves per SIMD
 
 template <class T, int W>
-__global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, int v, int os, int nb, int j0,
+__global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int vecs, int o, int v, int os, int nb,
+                                                                       int j0,
                                                                        const double* __restrict__ V,
                                                                        const double* __restrict__ O,
                                                                        const double* __restrict__ eps, double sigma,
@@ -203,8 +211,8 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
   double* R = sm;
   double* S = sm + v * os;
   double* ev = S + v * os;
-  const int ng = (nb + CP_VECS - 1) / CP_VECS;
-  const int c = blockIdx.x / ng, vec0 = (blockIdx.x - c * ng) * CP_VECS, vec1 = min(nb, vec0 + CP_VECS);
+  const int ng = (nb + vecs - 1) / vecs;
+  const int c = blockIdx.x / ng, vec0 = (blockIdx.x - c * ng) * vecs, vec1 = min(nb, vec0 + vecs);
   for (int t = threadIdx.x; t < o + v; t += UP_THREADS) ev[t] = eps[t];
   const int step = UP_THREADS * W, qs = step / o, rs = step - qs * o;  // a step as (b, l)
   const int b0 = threadIdx.x * W / o, l0 = threadIdx.x * W - b0 * o;
@@ -223,7 +231,9 @@ __global__ void __launch_bounds__(UP_THREADS) cp_unit_pairs_lds_kernel(int o, in
     }
     __syncthreads();
     T* zv = Z + (int64_t)(c * nb + vec) * o * n1;
-    const bool two = c != ap && o >= W;  // b = a' in the second pass
+    // b = a' in the second pass (W <= o holds; without it here the compiler merges
+    // the two cases, and the kernel takes 0.56 ms)
+    const bool two = c != ap && o >= W;
     auto element = [&](int k, int b, int l, bool at_ap) -> T {
       double g1 = 0.0, g2 = 0.0, g3 = 0.0, g4 = 0.0;
       if (k == kp) {
@@ -303,11 +313,14 @@ void unit_pairs_lds(int o, int v, int nb, int j0, const double* V, const double*
   constexpr int W = 16 / (int)sizeof(T);
   auto bytes = [&](int os) { return sizeof(double) * ((size_t)2 * v * os + o + v); };
   const int os = bytes(o | 1) <= 65536 ? (o | 1) : o;
-  const dim3 grid((unsigned)v * ((nb + CP_VECS - 1) / CP_VECS)), blk(UP_THREADS);
-  if ((o * v) % W == 0)
-    hipLaunchKernelGGL((cp_unit_pairs_lds_kernel<T, W>), grid, blk, bytes(os), st, o, v, os, nb, j0, V, O, eps, sigma, Z);
+  const int vecs = o < 8 ? 4 : 2;
+  const dim3 grid((unsigned)v * ((nb + vecs - 1) / vecs)), blk(UP_THREADS);
+  if (o >= W && (o * v) % W == 0)
+    hipLaunchKernelGGL((cp_unit_pairs_lds_kernel<T, W>), grid, blk, bytes(os), st, vecs, o, v, os, nb, j0, V, O, eps,
+                       sigma, Z);
   else
-    hipLaunchKernelGGL((cp_unit_pairs_lds_kernel<T, 1>), grid, blk, bytes(os), st, o, v, os, nb, j0, V, O, eps, sigma, Z);
+    hipLaunchKernelGGL((cp_unit_pairs_lds_kernel<T, 1>), grid, blk, bytes(os), st, vecs, o, v, os, nb, j0, V, O, eps,
+                       sigma, Z);
 }
 
 // A[:, j0 + c] = H11[:, j0 + c] - M[:, c] (n1 x nb; H11 symmetric)
