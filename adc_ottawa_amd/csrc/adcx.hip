@@ -148,23 +148,35 @@ __global__ void ax_kpm_kernel(const double* __restrict__ I, DimsK d, int64_t ldp
   }
 }
 
-// Op[(k<=l)][(m<=n)] = (km|ln) + (kn|lm) (m < n), (km|lm) (m = n); Om with a
-// minus sign and no equal pairs.  oooo[(m,n)][(k,l)] = (km|ln).
+// Columns of the matrices of the occupied ladder: whole blocks of ax_ladder_kernel.
+constexpr int AX_LADDER_ROWS = 64;
+__host__ __device__ __forceinline__ int ax_ladder_ld(int64_t n) {
+  return (int)((n + AX_LADDER_ROWS - 1) / AX_LADDER_ROWS) * AX_LADDER_ROWS;
+}
+
+// Op[(m<=n)][(k<=l)] = (km|ln) + (kn|lm) (m < n), (km|lm) (m = n); Om with a
+// minus sign and no equal pairs: rows of ax_ladder_ld elements, zero rows and
+// columns up to as many.  oooo[(m,n)][(k,l)] = (km|ln).
 __global__ void ax_opm_kernel(const double* __restrict__ oooo, DimsK d, double* __restrict__ Op,
                               double* __restrict__ Om) {
   const int o = d.o;
-  const int64_t so = d.npo + o;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < so * so;
+  const int64_t so = d.npo + o, lp = ax_ladder_ld(so), lm = ax_ladder_ld(d.npo);
+  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < lp * lp;
        idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = idx / so, q = idx - r * so;
-    int k, l, m, n;
-    if (r < d.npo) ax_unpair(r, o, k, l);
-    else k = l = (int)(r - d.npo);
-    if (q < d.npo) ax_unpair(q, o, m, n);
-    else m = n = (int)(q - d.npo);
-    const double g1 = oooo[(((int64_t)m * o + n) * o + k) * o + l], g2 = oooo[(((int64_t)n * o + m) * o + k) * o + l];
-    Op[idx] = m == n ? g1 : g1 + g2;
-    if (r < d.npo && q < d.npo) Om[r * d.npo + q] = g1 - g2;
+    const int64_t q = idx / lp, r = idx - q * lp;
+    double p = 0.0, x = 0.0;
+    if (r < so && q < so) {
+      int k, l, m, n;
+      if (r < d.npo) ax_unpair(r, o, k, l);
+      else k = l = (int)(r - d.npo);
+      if (q < d.npo) ax_unpair(q, o, m, n);
+      else m = n = (int)(q - d.npo);
+      const double g1 = oooo[(((int64_t)m * o + n) * o + k) * o + l], g2 = oooo[(((int64_t)n * o + m) * o + k) * o + l];
+      p = m == n ? g1 : g1 + g2;
+      x = r < d.npo && q < d.npo ? g1 - g2 : 0.0;
+    }
+    Op[idx] = p;
+    if (r < lm && q < lm) Om[q * lm + r] = x;
   }
 }
 
@@ -232,34 +244,92 @@ __global__ void ax_project_kernel(const double* __restrict__ G1, const double* _
   }
 }
 
-// the ladder terms: w4 += sqrt2 S+, w3 += S+, w2 -= S+, w1 -= S+ / sqrt2, w5 +=
-// S- (already in units of x5), rows as in ax_pm_kernel
-__global__ void ax_ladder_kernel(const double* __restrict__ Sp, const double* __restrict__ Sm, int nb, DimsK d,
-                                 int64_t ldp, int64_t ldm, double* __restrict__ W, int64_t ldw) {
+// The occupied ladder added to the virtual one in S+ (PLUS) or S-, and both to
+// the CSFs: w4 += sqrt2 S+, w3 += S+, w2 -= S+, w1 -= S+ / sqrt2, w5 += S-
+// (already in units of x5); rows as in ax_pm_kernel, ld elements each.  A
+// workgroup takes 16 columns p and 64 rows kl on FP64 MFMA, its four waves every
+// fourth run of 16 pairs mn (one wave alone is a chain of (o/2)^2 / 8 round trips to
+// the L2); T is read along p and the matrix along kl, whole cache lines both, and
+// S is read once.  As products of their own (three launches of few workgroups) the
+// occupied terms and the addition took 67 us of the 200 of one vector at o=12,
+// v=24; this kernel 8.5.
+constexpr int AX_MB = AX_LADDER_ROWS / 16;
+static_assert(AX_MB == 4, "one block of rows for each wave at the end");
+
+template <bool PLUS>
+__device__ __forceinline__ void ax_ladder(const double* __restrict__ T, const double* __restrict__ O,
+                                          const double* __restrict__ S, const DimsK& d, int64_t ld, int chunk,
+                                          double* __restrict__ W, int64_t ldw,
+                                          double (*red)[AX_MB][4][64]) {  // [wave][block][register][lane]
+  typedef Mma<double> MT;
+  typedef MT::v4 v4;
+  constexpr int MB = AX_MB;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, gq = lane >> 4;
+  const int64_t npv = d.npv;
+  const int n = (int)(PLUS ? d.npo + d.o : d.npo), lo = ax_ladder_ld(n);
+  const int64_t j = blockIdx.y, p = (int64_t)blockIdx.x * 16 + li;
+  const int kl0 = chunk * AX_LADDER_ROWS;
+  if (p - li >= ld) return;  // the whole workgroup (ld is a multiple of 16)
+  const double* t = T + j * n * ld + p;
+  const double* a = O + kl0 + li;
+  v4 acc[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) acc[m] = (v4){0, 0, 0, 0};
+  for (int k = wv * 16; k < n; k += 64) {
+    double b[4], x[4][MB];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int mn = k + 4 * s + gq;  // (rows past n: zeros)
+      b[s] = t[min(mn, n - 1) * ld];
+      b[s] = mn < n ? b[s] : 0.0;
+#pragma unroll
+      for (int m = 0; m < MB; ++m) x[s][m] = a[(int64_t)mn * lo + m * 16];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) acc[m] = MT::mma(x[s][m], b[s], acc[m]);
+  }
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wv][m][r][lane] = acc[m][r];
+  __syncthreads();
   const int o = d.o, v = d.v;
-  const int64_t so = d.npo + o;
-  const int64_t row = blockIdx.y + (int64_t)gridDim.y * blockIdx.z;
-  if (row >= so * nb) return;
-  const int64_t j = row / so, kl = row - j * so;
+  if (p >= (PLUS ? npv + v : npv)) return;
+  const double* s0 = S + j * n * ld + p;
   double* w = W + ldw * j;
-  const double* sp = Sp + row * ldp;
-  const double* sm = Sm + (j * d.npo + kl) * ldm;
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < d.npv + v;
-       p += (int64_t)gridDim.x * blockDim.x) {
-    const double s = sp[p];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t kl = kl0 + wv * 16 + MT::row(lane, r);
+    if (kl >= n) continue;
+    const double occ = (red[0][wv][r][lane] + red[1][wv][r][lane]) + (red[2][wv][r][lane] + red[3][wv][r][lane]);
+    if (!PLUS) {
+      w[d.off5 + kl * npv + p] += s0[kl * ld] + occ;
+      continue;
+    }
+    // (T+ of c = b is not doubled)
+    const double s = s0[kl * ld] + (p < npv ? 0.5 : 1.0) * occ;
     if (kl < d.npo) {
-      if (p < d.npv) {
-        w[d.off4 + kl * d.npv + p] += AX_SQ2 * s;
-        w[d.off5 + kl * d.npv + p] += sm[p];
-      } else {
-        w[d.off3 + kl * v + p - d.npv] += s;
-      }
+      if (p < npv) w[d.off4 + kl * npv + p] += AX_SQ2 * s;
+      else w[d.off3 + kl * v + p - npv] += s;
     } else {
       const int64_t k = kl - d.npo;
-      if (p < d.npv) w[d.off2 + p * o + k] -= s;
-      else w[d.off1 + k * v + p - d.npv] -= AX_ISQ2 * s;
+      if (p < npv) w[d.off2 + p * o + k] -= s;
+      else w[d.off1 + k * v + p - npv] -= AX_ISQ2 * s;
     }
   }
+}
+
+// workgroups (columns, vector, rows): the first cp of the rows S+, the others S-
+__global__ void __launch_bounds__(256)
+ax_ladder_kernel(const double* __restrict__ Tp, const double* __restrict__ Op, const double* __restrict__ Sp,
+                 const double* __restrict__ Tm, const double* __restrict__ Om, const double* __restrict__ Sm, DimsK d,
+                 int64_t ldp, int64_t ldm, int cp, double* __restrict__ W, int64_t ldw) {
+  __shared__ double red[4][AX_MB][4][64];
+  const int z = blockIdx.z;
+  if (z < cp) ax_ladder<true>(Tp, Op, Sp, d, ldp, z, W, ldw, red);
+  else ax_ladder<false>(Tm, Om, Sm, d, ldm, z - cp, W, ldw, red);
 }
 
 struct AxMats {
@@ -450,10 +520,10 @@ void Handle::enable_adcx(bool on) {
       launch_transpose<double, double>(R.get(), oo, oo, ax_oooo.get(), st);
       HIP_CHECK(hipStreamSynchronize(st));
     }
-    const int64_t so = d.npo + o;
-    ax_op.alloc((size_t)so * so);
-    ax_om.alloc((size_t)d.npo * d.npo);
-    hipLaunchKernelGGL(ax_opm_kernel, dim3(grid_for(so * so)), dim3(256), 0, st, ax_oooo.get(), dk, ax_op.get(),
+    const int64_t lp = ax_ladder_ld(d.npo + o), lm = ax_ladder_ld(d.npo);
+    ax_op.alloc((size_t)lp * lp);
+    ax_om.alloc((size_t)lm * lm);
+    hipLaunchKernelGGL(ax_opm_kernel, dim3(grid_for(lp * lp)), dim3(256), 0, st, ax_oooo.get(), dk, ax_op.get(),
                        ax_om.get());
     HIP_CHECK(hipGetLastError());
     ax_d2.alloc((size_t)n2);
@@ -522,20 +592,10 @@ void Handle::adcx_apply(const double* X, int64_t ldx, double* W, int64_t ldw, in
                0.0, s);
     ax_gemm_bt(*this, (int)(nb * d.npo), (int)d.npv, (int)ldm, ax_tm.get(), ldm, ax_km.get(), ldm, ax_sm.get(), ldm,
                1.0, 0.0, s);
-    auto occ = [&](const double* O, int64_t n, const double* T, int64_t ld, double* S, int64_t col0, int64_t ncol,
-                   double alpha) {  // S[(j,kl)][cb] += alpha O[kl][mn] T[(j,mn)][cb]
-      if (ncol <= 0) return;
-      GemmArgs g;
-      g.M = (int)n; g.N = (int)ncol; g.K = (int)n; g.batch = nb;
-      g.A = O; g.sam = n; g.sak = 1; g.sab = 0;
-      g.B = T + col0; g.sbk = ld; g.sbn = 1; g.sbb = n * ld;
-      g.map.C = S + col0; g.map.scm = ld; g.map.scn = 1; g.map.scb = n * ld; g.map.alpha = alpha; g.map.beta = 1.0;
-      gemm(g, Prec::F64, gws, s);
-    };
-    occ(ax_op.get(), so, ax_tp.get(), ldp, ax_sp.get(), 0, d.npv, 0.5);
-    occ(ax_op.get(), so, ax_tp.get(), ldp, ax_sp.get(), d.npv, v, 1.0);  // (T+ of c = b is not doubled)
-    occ(ax_om.get(), d.npo, ax_tm.get(), ldm, ax_sm.get(), 0, d.npv, 1.0);
-    hipLaunchKernelGGL(ax_ladder_kernel, rows, dim3(256), 0, s, ax_sp.get(), ax_sm.get(), nb, dk, ldp, ldm, w, ldw);
+    const int cp = ax_ladder_ld(so) / AX_LADDER_ROWS, cm = ax_ladder_ld(d.npo) / AX_LADDER_ROWS;
+    hipLaunchKernelGGL(ax_ladder_kernel, dim3((unsigned)(ldp / 16), (unsigned)nb, (unsigned)(cp + cm)), dim3(256), 0, s,
+                       ax_tp.get(), ax_op.get(), ax_sp.get(), ax_tm.get(), ax_om.get(), ax_sm.get(), dk, ldp, ldm, cp,
+                       w, ldw);
     HIP_CHECK(hipGetLastError());
   }
 }

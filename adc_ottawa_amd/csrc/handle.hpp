@@ -136,7 +136,7 @@ struct Handle {
   // ADC(2)-x: the first-order 2h2p-2h2p block added to the sigma-vector
   // (FP64) and its diagonal to hii.  Integral matrices (built on enable):
   // ax_kp, ax_km [(c<=b)][(d<=e)] = (cd|be) +- (ce|bd), ax_op, ax_om the same of
-  // (oo|oo), ax_ov [(c,k)][(d,m)] = (ck|dm), ax_vo [(c,k)][(d,m)] = (cd|km), ax_a1
+  // (oo|oo) transposed, ax_ov [(c,k)][(d,m)] = (ck|dm), ax_vo [(c,k)][(d,m)] = (cd|km), ax_a1
   // = 2 ax_ov - ax_vo; per-chunk layouts of T and partial results (adcx.hip).
   bool adcx = false;
   DevBuf<double> ax_kp, ax_km, ax_op, ax_om, ax_ov, ax_vo, ax_a1, ax_d2;
