@@ -55,9 +55,10 @@ def test_adcx_sigma_and_diagonal(form, o, v, naux, seed):
 
 # runs of pairs that leave a remainder in the tiled ring layouts (16 virtuals a run
 # at few occupied orbitals, one at 64), the element-wise layouts beyond 64, padded
-# and whole rows of the ladder products, and (19 vectors) a second chunk of vectors
+# and whole rows of the ladder products, one and two runs of 64 occupied pairs on
+# either side of the line, and (19 vectors) a second chunk of vectors
 @pytest.mark.parametrize("o,v,nvec", [(2, 2, 1), (3, 20, 19), (4, 37, 2), (2, 33, 17), (9, 18, 3), (33, 5, 2),
-                                      (64, 2, 2), (65, 2, 2), (66, 4, 2)])
+                                      (11, 6, 2), (12, 14, 2), (64, 2, 2), (65, 2, 2), (66, 4, 2)])
 def test_adcx_sigma_edges(o, v, nvec):
     print(f"[case] adcx sigma edges o={o} v={v} nvec={nvec}", flush=True)
     sys_ = make_system(o, v, 12, seed=o + v)
